@@ -36,6 +36,7 @@
 //     four LDS stages (buffer_load ... lds, three steps ahead), because the
 //     32-byte fp8 fragments leave no registers for load staging.
 #include <atomic>
+#include <cmath>
 
 #include "hmoe_common.h"
 
@@ -1199,6 +1200,476 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_regs(
   }
 }
 
+// 16 bytes a lane from byte voff + soff of the resource to the uniform LDS
+// address dst + 16 lane, and the e4m3 MFMA with A's block exponents (byte 2 q of
+// ex).  Functions of their own: written inside a kernel template, where their
+// arguments are dependent, the host pass drops the kernel's stub.
+__device__ __forceinline__ void few_dma16(__amdgpu_buffer_rsrc_t r, uint8_t* dst, uint32_t voff,
+                                          int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ void few_dma4(__amdgpu_buffer_rsrc_t r, uint8_t* dst, uint32_t voff,
+                                         int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 4, voff, soff, 0, 0);
+}
+__device__ __forceinline__ f32x16 few_mfma_scaled(const i32x8& b, const i32x8& a, const f32x16& c,
+                                                  int ex, int q) {
+  if (q == 0) return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b, a, c, 0, 0, 0, 127, 0, ex);
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b, a, c, 0, 0, 0, 127, 2, ex);
+}
+// ---- few rows per expert -----------------------------------------------------
+// The grouped GEMMs when the experts have too few rows for 256 x 256 tiles (a
+// decode step, a short prompt, a small training batch, one shared expert).  The
+// weights then dominate what is read, so the kernel is built to stream them: a
+// BM x BN tile per workgroup (4 waves), K steps of 128 bytes of every A and B
+// row that go straight from global memory into a ring of kStages LDS stages
+// (buffer_load ... lds, 16 bytes a lane, eight lanes a row; chunk c of row r at
+// c ^ lds_swz(r)), kStages - 1 steps ahead across tile boundaries, one barrier
+// per step.  About 100 KB of every CU's LDS is in flight at a time; nothing in
+// the loop waits for memory but the ring itself: the tile table and the offsets
+// are in LDS and the gathered rows' sources come through scalar loads, which
+// do not count in vmcnt.  Wave w computes columns 64 (w % kWN) .. + 64 (a gate
+// and an up block) of every kWM-th 32-row fragment; with fewer fragments than
+// waves the others only load.  Tiles are numbered and dealt to the XCDs as in
+// the 256 x 256 kernels, and every output is summed in the same K order, so
+// the results are the same bits.
+enum FewEpi { kFewPlain = 0, kFewSwiglu = 1, kFewDSwiglu = 2, kFewSwigluQ = 3 };
+enum FewElem { kFewBf16 = 0, kFewE4m3 = 1, kFewE4m3Mx = 2 };  // Mx: block-scaled A
+
+template <int ELEM, int BM, int BN>
+struct FewCfg {
+  static constexpr int kExBytes = ELEM == kFewE4m3Mx ? BM * 4 < 256 ? 256 : BM * 4 : 0;
+  static constexpr int kStage = (BM + BN) * 128 + kExBytes;
+  static constexpr int kFit = 150 * 1024 / kStage;
+  static constexpr int kStages = kFit < 12 ? kFit : 12;
+  static constexpr int kLds = kStages * kStage;
+  static constexpr int kNA = BM / 32, kNB = BN / 32;  // DMA instructions per wave and step
+  static_assert(kStages >= 3, "the ring needs three stages");
+  static_assert((kStages - 2) * (kNA + kNB) < 63, "vmcnt is a 6-bit count");
+};
+
+template <int BM>
+__device__ __forceinline__ int scan_few_tiles(const int32_t* __restrict__ offsets, int n_experts,
+                                              int32_t* toff, int32_t* tstart, int32_t* scan_tmp) {
+  const int tid = threadIdx.x;
+  const int per = (n_experts + kThreads - 1) / kThreads;
+  for (int e = tid; e <= n_experts; e += kThreads) toff[e] = offsets[e];
+  __syncthreads();
+  int sum = 0;
+  for (int j = 0; j < per; ++j) {
+    const int e = tid * per + j;
+    if (e < n_experts) sum += (toff[e + 1] - toff[e] + BM - 1) / BM;
+  }
+  scan_tmp[tid] = sum;
+  __syncthreads();
+  for (int off = 1; off < kThreads; off <<= 1) {
+    const int v = tid >= off ? scan_tmp[tid - off] : 0;
+    __syncthreads();
+    scan_tmp[tid] += v;
+    __syncthreads();
+  }
+  int run = scan_tmp[tid] - sum;
+  for (int j = 0; j < per; ++j) {
+    const int e = tid * per + j;
+    if (e < n_experts) {
+      tstart[e] = run;
+      run += (toff[e + 1] - toff[e] + BM - 1) / BM;
+    }
+  }
+  if (tid == kThreads - 1) tstart[n_experts] = scan_tmp[kThreads - 1];
+  __syncthreads();
+  return tstart[n_experts];
+}
+
+template <int ELEM, int EPI, bool GATHER, int BM, int BN>
+__global__ __launch_bounds__(kThreads) void grouped_gemm_few(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
+    const float* __restrict__ a_scale, const float* __restrict__ b_scale,
+    const int32_t* __restrict__ offsets, int n_experts, int kdim, int ncols,
+    uint16_t* __restrict__ C, int64_t ldc, const int32_t* __restrict__ gather_src, int gather_k,
+    int gather_rows, const uint16_t* __restrict__ dh, uint8_t* __restrict__ mx_exp) {
+  typedef FewCfg<ELEM, BM, BN> Cfg;
+  constexpr bool kFp8 = ELEM != kFewBf16;
+  constexpr int kNA = Cfg::kNA, kNB = Cfg::kNB, kStages = Cfg::kStages;
+  constexpr int kWN = BN / 64;                             // column groups of waves
+  constexpr int kWM = 4 / kWN;                             // row groups
+  constexpr int kRB = BM / 32;
+  constexpr int kFR = kRB >= kWM ? kRB / kWM : 1;          // row fragments per wave
+  static_assert(!(ELEM == kFewE4m3Mx && GATHER), "the block-scaled A operand is not gathered");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  __shared__ int32_t toff[kMaxExperts + 1];
+  __shared__ int32_t tstart[kMaxExperts + 1];
+  __shared__ int32_t scan_tmp[kThreads];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_tiles_n = ncols / BN;
+  const int total = __builtin_amdgcn_readfirstlane(
+      scan_few_tiles<BM>(offsets, n_experts, toff, tstart, scan_tmp) * n_tiles_n);
+  const int xcd = blockIdx.x % kNumXcd;
+  const int per_xcd = gridDim.x / kNumXcd;
+  const int slot = blockIdx.x / kNumXcd;
+  const int lo = static_cast<int>((static_cast<int64_t>(total) * xcd) / kNumXcd);
+  const int hi = static_cast<int>((static_cast<int64_t>(total) * (xcd + 1)) / kNumXcd);
+  const int first = lo + slot;
+  if (first >= hi) return;  // uniform per workgroup
+  const int row_bytes = kFp8 ? kdim : kdim * 2;
+  const int ks = row_bytes / 128;
+  const int iters = (hi - first + per_xcd - 1) / per_xcd * ks;
+
+  // Tile t: as decode_tile_grouped (groups of 8 row tiles, row tile fastest).
+  struct Tile {
+    int e, row0, row_end, n0;
+  };
+  auto decode = [&](int t) __attribute__((always_inline)) {
+    constexpr int G = 8;
+    const int m_any = t / n_tiles_n;
+    int l = 0, h = n_experts;
+    while (h - l > 1) {
+      const int mid = (l + h) >> 1;
+      if (tstart[mid] <= m_any) l = mid; else h = mid;
+    }
+    const int e = __builtin_amdgcn_readfirstlane(l);
+    const int ts = __builtin_amdgcn_readfirstlane(tstart[e]);
+    const int me = __builtin_amdgcn_readfirstlane(tstart[e + 1]) - ts;
+    const int u = t - ts * n_tiles_n;
+    const int g = u / (G * n_tiles_n);
+    const int gm = me - g * G < G ? me - g * G : G;
+    const int v = u - g * G * n_tiles_n;
+    const int n_tile = v / gm;
+    Tile r;
+    r.e = e;
+    r.row0 = __builtin_amdgcn_readfirstlane(toff[e]) + (g * G + (v - n_tile * gm)) * BM;
+    r.row_end = __builtin_amdgcn_readfirstlane(toff[e + 1]);
+    r.n0 = n_tile * BN;
+    return r;
+  };
+
+  // ---- load side ---------------------------------------------------------------
+  // Instruction j of wave w fills rows 8 (w kNA + j) + lane / 8 of A's part of
+  // a stage (B's alike with kNB), lane position lane % 8.
+  const int l8 = lane >> 3;
+  uint32_t a_voff[kNA], b_voff[kNB];
+#pragma unroll
+  for (int j = 0; j < kNB; ++j) {
+    const int row = 8 * (wave * kNB + j) + l8;
+    b_voff[j] = static_cast<uint32_t>(row * row_bytes + ((lane & 7) ^ lds_swz(row)) * 16);
+  }
+  __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(A), 0, GATHER ? gather_rows * row_bytes : 0, kBufferWord3);
+  __amdgpu_buffer_rsrc_t b_rsrc = a_rsrc, e_rsrc = a_rsrc;
+  uint32_t e_voff = 0;
+  int ld_t = first, ld_kb = 0, ld_g = 0, ld_slot = 0;
+  auto set_load_tile = [&](int t) __attribute__((always_inline)) {
+    const Tile q = decode(t);
+    b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(B + (static_cast<int64_t>(q.e) * ncols + q.n0) * row_bytes), 0,
+        BN * row_bytes, kBufferWord3);
+    const int lim = q.row_end - 1 - q.row0;  // rows past the segment repeat its last one
+    if constexpr (GATHER) {
+      typedef const __attribute__((address_space(4))) int32_t* scalar_ptr;
+      const scalar_ptr src = (scalar_ptr)(uintptr_t)gather_src;
+#pragma unroll
+      for (int j = 0; j < kNA; ++j) {
+        const int r = 8 * (wave * kNA + j);
+        int s = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int si = src[q.row0 + (r + i < lim ? r + i : lim)];
+          s = l8 == i ? si : s;
+        }
+        int tk = s >= 0 ? s / gather_k : 0;  // a row without a source reads token 0
+        tk = tk < gather_rows ? tk : gather_rows - 1;
+        a_voff[j] = gather_offset(tk, row_bytes, ((lane & 7) ^ lds_swz(r + l8)) * 16);
+      }
+    } else {
+      a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint8_t*>(A + static_cast<int64_t>(q.row0) * row_bytes), 0,
+          (lim < BM ? lim + 1 : BM) * row_bytes, kBufferWord3);
+#pragma unroll
+      for (int j = 0; j < kNA; ++j) {
+        const int r = 8 * (wave * kNA + j) + l8;
+        a_voff[j] = static_cast<uint32_t>((r < lim ? r : lim) * row_bytes +
+                                          ((lane & 7) ^ lds_swz(r)) * 16);
+      }
+    }
+    if constexpr (ELEM == kFewE4m3Mx) {
+      const int ex_bytes = kdim / 32;
+      e_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          mx_exp + static_cast<int64_t>(q.row0) * ex_bytes, 0, (lim < BM ? lim + 1 : BM) * ex_bytes,
+          kBufferWord3);
+      const int r = (wave * 64 + lane) % BM;
+      e_voff = static_cast<uint32_t>((r < lim ? r : lim) * ex_bytes);
+    }
+  };
+  auto issue = [&]() __attribute__((always_inline)) {
+    uint8_t* st = smem + ld_slot * Cfg::kStage;
+    const int koff = ld_kb * 128;
+    if constexpr (ELEM == kFewE4m3Mx) {
+      // the 4 exponents of every row's step, by the first waves
+      if (wave < (BM + 63) / 64)
+        few_dma4(e_rsrc, st + (BM + BN) * 128 + wave * 256, e_voff, ld_kb * 4);
+    }
+#pragma unroll
+    for (int j = 0; j < kNA; ++j) few_dma16(a_rsrc, st + (wave * kNA + j) * 1024, a_voff[j], koff);
+#pragma unroll
+    for (int j = 0; j < kNB; ++j)
+      few_dma16(b_rsrc, st + BM * 128 + (wave * kNB + j) * 1024, b_voff[j], koff);
+    ld_slot = ld_slot + 1 == kStages ? 0 : ld_slot + 1;
+    ++ld_g;
+    if (++ld_kb == ks) {
+      ld_kb = 0;
+      ld_t += per_xcd;
+      if (ld_t < hi) set_load_tile(ld_t);
+    }
+  };
+
+  // ---- compute side --------------------------------------------------------------
+  const int wn = wave % kWN, wm = wave / kWN;
+  const bool active = wm < kRB;  // uniform per wave
+  const int frow = lane & 31, fhalf = lane >> 5;
+  f32x16 acc[kFR][2];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kFR; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+  };
+  // Fragment i of a wave: tile rows 32 (wm + kWM i) .. + 32.
+  auto compute = [&](int sl) __attribute__((always_inline)) {
+    const uint8_t* st = smem + sl * Cfg::kStage;
+    const uint8_t* sb = st + BM * 128 + wn * 64 * 128;
+    if constexpr (!kFp8) {
+      typedef GemmElem<false> E;
+#pragma unroll
+      for (int q = 0; q < E::kSub; ++q) {
+        E::frag_t fa[kFR], fb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[j] = E::read(sb, (32 * j + frow) * 128, frow, q, fhalf);
+#pragma unroll
+        for (int i = 0; i < kFR; ++i)
+          fa[i] = E::read(st, (32 * (wm + kWM * i) + frow) * 128, frow, q, fhalf);
+#pragma unroll
+        for (int i = 0; i < kFR; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = E::mfma(fb[j], fa[i], acc[i][j]);
+      }
+    } else {
+      typedef GemmElem<true> E;
+      const int sw = lds_swz(frow);
+      auto read = [&](const uint8_t* row, int q) __attribute__((always_inline)) {
+        const u32x4 lo4 = *reinterpret_cast<const u32x4*>(row + ((4 * q + fhalf) ^ sw) * 16);
+        const u32x4 hi4 = *reinterpret_cast<const u32x4*>(row + ((4 * q + 2 + fhalf) ^ sw) * 16);
+        E::frag_t f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          f[w] = static_cast<int>(lo4[w]);
+          f[4 + w] = static_cast<int>(hi4[w]);
+        }
+        return f;
+      };
+      int ex[kFR];
+      if constexpr (ELEM == kFewE4m3Mx) {
+        // byte 2 q of the shifted word is this lane's block of sub-step q
+#pragma unroll
+        for (int i = 0; i < kFR; ++i)
+          ex[i] = static_cast<int>(*reinterpret_cast<const uint32_t*>(
+                                       st + (BM + BN) * 128 + (32 * (wm + kWM * i) + frow) * 4) >>
+                                   (8 * fhalf));
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        E::frag_t fa[kFR], fb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[j] = read(sb + (32 * j + frow) * 128, q);
+#pragma unroll
+        for (int i = 0; i < kFR; ++i) fa[i] = read(st + (32 * (wm + kWM * i) + frow) * 128, q);
+#pragma unroll
+        for (int i = 0; i < kFR; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            if constexpr (ELEM == kFewE4m3Mx)
+              acc[i][j] = few_mfma_scaled(fb[j], fa[i], acc[i][j], ex[i], q);
+            else
+              acc[i][j] = E::mfma(fb[j], fa[i], acc[i][j]);
+          }
+      }
+    }
+  };
+
+  // Epilogue: lane L of acc[i][j] holds its fragment's row L % 32 and columns
+  // 64 wn + 32 j + 8 q + 4 (L / 32) + 0..3 of the tile; lanes L and L + 32 trade
+  // groups so that every store is 16 bytes, two a row and block.  The stores'
+  // range ends at the segment's last row.
+  auto epilogue = [&](const Tile& q) __attribute__((always_inline)) {
+    constexpr int kOutB = EPI == kFewSwigluQ ? 1 : 2;
+    const int nrows = q.row_end - q.row0 < BM ? q.row_end - q.row0 : BM;
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<uint8_t*>(C) + static_cast<int64_t>(q.row0) * ldc * kOutB, 0,
+        static_cast<int>(nrows * ldc * kOutB), kBufferWord3);
+    auto store_block = [&](uint32_t (&d)[8], int r, int col) __attribute__((always_inline)) {
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const auto p01 = __builtin_amdgcn_permlane32_swap(d[w], d[2 + w], false, false);
+        d[w] = p01[0];
+        d[2 + w] = p01[1];
+        const auto p23 = __builtin_amdgcn_permlane32_swap(d[4 + w], d[6 + w], false, false);
+        d[4 + w] = p23[0];
+        d[6 + w] = p23[1];
+      }
+      const int off = static_cast<int>((r * ldc + col + fhalf * 8) * 2);
+      const u32x4 lo4 = {d[0], d[1], d[2], d[3]};
+      const u32x4 hi4 = {d[4], d[5], d[6], d[7]};
+      __builtin_amdgcn_raw_buffer_store_b128(lo4, c_rsrc, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(hi4, c_rsrc, off + 32, 0, 0);
+    };
+    f32x4 sc[2][4];  // column scales of this lane's groups
+    if constexpr (kFp8) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          sc[j][w] = *reinterpret_cast<const f32x4*>(b_scale + static_cast<int64_t>(q.e) * ncols + q.n0 +
+                                                     wn * 64 + 32 * j + 8 * w + 4 * fhalf);
+    }
+#pragma unroll
+    for (int i = 0; i < kFR; ++i) {
+      const int r = 32 * (wm + kWM * i) + frow;
+      float sa = 1.0f;  // (block-scaled A: inside the MFMA)
+      if constexpr (ELEM == kFewE4m3) {
+        const int rr = q.row0 + (r < nrows ? r : nrows - 1);
+        if (GATHER) {
+          const int s = gather_src[rr];
+          int tk = s >= 0 ? s / gather_k : 0;
+          tk = tk < gather_rows ? tk : gather_rows - 1;
+          sa = a_scale[tk];
+        } else {
+          sa = a_scale[rr];
+        }
+      }
+      if constexpr (kFp8) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int k = 0; k < 16; ++k) acc[i][j][k] = acc[i][j][k] * sa * sc[j][k >> 2][k & 3];
+      }
+      const int hcol = q.n0 / 2 + wn * 32;
+      if constexpr (EPI == kFewSwigluQ) {
+        // as the 256 x 256 kernel: block maximum over lanes L and L + 32, the
+        // smallest exponent that covers it, codes and the biased exponent
+        float hv[16];
+        float amax = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; k += 2) {
+          const uint32_t pk = pack_bf16x2_rne(swiglu_bf16_points(acc[i][0][k], acc[i][1][k]),
+                                              swiglu_bf16_points(acc[i][0][k + 1], acc[i][1][k + 1]));
+          hv[k] = __uint_as_float(pk << 16);
+          hv[k + 1] = __uint_as_float(pk & 0xffff0000u);
+          amax = fmaxf(amax, fmaxf(fabsf(hv[k]), fabsf(hv[k + 1])));
+        }
+        const uint32_t abits = __float_as_uint(amax);
+        const auto pa = __builtin_amdgcn_permlane32_swap(abits, abits, false, false);
+        const uint32_t bmax = __float_as_uint(fmaxf(__uint_as_float(pa[0]), __uint_as_float(pa[1])));
+        int ex = static_cast<int>(bmax >> 23) - 135 + ((bmax & 0x7FFFFFu) > 0x600000u ? 1 : 0);
+        ex = ex > -127 ? ex : -127;
+        const float inv = __uint_as_float(static_cast<uint32_t>(127 - ex) << 23);
+        uint32_t d[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          float v[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] = fminf(fmaxf(hv[w * 4 + k] * inv, -448.0f), 448.0f);
+          const int lo2 = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
+          d[w] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], lo2, true));
+        }
+        const auto p02 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
+        const auto p13 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+        const u32x4 codes = {p02[0], p02[1], p13[0], p13[1]};
+        __builtin_amdgcn_raw_buffer_store_b128(codes, c_rsrc,
+                                               static_cast<int>(r * ldc + hcol + 16 * fhalf), 0, 0);
+        const __amdgpu_buffer_rsrc_t e_out = __builtin_amdgcn_make_buffer_rsrc(
+            mx_exp + static_cast<int64_t>(q.row0) * (ldc / 32), 0, static_cast<int>(nrows * (ldc / 32)),
+            kBufferWord3);
+        if (fhalf == 0)
+          __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(ex + 127), e_out,
+                                               static_cast<int>(r * (ldc / 32) + hcol / 32), 0, 0);
+      } else if constexpr (EPI == kFewSwiglu) {
+        uint32_t d[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          d[k] = pack_bf16x2_rne(swiglu_bf16_points(acc[i][0][2 * k], acc[i][1][2 * k]),
+                                 swiglu_bf16_points(acc[i][0][2 * k + 1], acc[i][1][2 * k + 1]));
+        store_block(d, r, hcol);
+      } else if constexpr (EPI == kFewDSwiglu) {
+        const int f = static_cast<int>(ldc / 2);
+        const __amdgpu_buffer_rsrc_t dh_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(dh + static_cast<int64_t>(q.row0) * f), 0, nrows * f * 2, kBufferWord3);
+        typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+        uint32_t dg[8], du[8];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const u32x2_t dv = __builtin_bit_cast(
+              u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(dh_rsrc, (r * f + hcol + 8 * w + 4 * fhalf) * 2,
+                                                            0, 0));
+          float vg[4], vu[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float d = __uint_as_float((k & 1) ? (dv[k >> 1] & 0xffff0000u) : (dv[k >> 1] << 16));
+            const uint32_t gu = pack_bf16x2_rne(acc[i][0][w * 4 + k], acc[i][1][w * 4 + k]);
+            swiglu_vjp(d, __uint_as_float(gu << 16), __uint_as_float(gu & 0xffff0000u), vg[k], vu[k]);
+          }
+          dg[2 * w] = pack_bf16x2_rne(vg[0], vg[1]);
+          dg[2 * w + 1] = pack_bf16x2_rne(vg[2], vg[3]);
+          du[2 * w] = pack_bf16x2_rne(vu[0], vu[1]);
+          du[2 * w + 1] = pack_bf16x2_rne(vu[2], vu[3]);
+        }
+        store_block(dg, r, q.n0 + wn * 64);
+        store_block(du, r, q.n0 + wn * 64 + 32);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          uint32_t d[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) d[k] = pack_bf16x2_rne(acc[i][j][2 * k], acc[i][j][2 * k + 1]);
+          store_block(d, r, q.n0 + wn * 64 + 32 * j);
+        }
+      }
+    }
+  };
+
+  set_load_tile(first);
+#pragma unroll 1
+  for (int i = 0; i < kStages - 1 && i < iters; ++i) issue();
+  clear();
+  int t = first, kb = 0, sl = 0;
+#pragma unroll 1
+  for (int g = 0; g < iters; ++g) {
+    // step g has landed (the waves' other kStages - 2 steps may still fly);
+    // after the barrier every wave's has, and every wave is done with step
+    // g - 1, whose stage the next loads take
+    if (ld_g < iters) {
+      wait_vm_lgkm0<(kStages - 2) * (kNA + kNB)>();
+      __builtin_amdgcn_s_barrier();
+      issue();
+    } else {
+      wait_vm_lgkm0<0>();
+      __builtin_amdgcn_s_barrier();
+    }
+    if (active) compute(sl);
+    sl = sl + 1 == kStages ? 0 : sl + 1;
+    if (++kb == ks) {
+      kb = 0;
+      if (active) {
+        epilogue(decode(t));
+        clear();
+      }
+      t += per_xcd;
+    }
+  }
+}
+
 // ---- weight gradients: ragged-K grouped GEMM -----------------------------------
 // C_e[m][n] = sum over the rows r of expert e's segment [offsets[e],
 // offsets[e+1]) of A[r][m] * B[r][n]: dWd[e] = h^T d_ys and dWg|dWu[e] =
@@ -1960,6 +2431,93 @@ int allow_dynamic_lds(int dev) {
   return HMOE_OK;
 }
 
+// The tile of a grouped GEMM over `rows` rows on n_experts experts: 256 x 256
+// (grouped_gemm_regs, grouped_gemm_w8_fp8) or one of grouped_gemm_few's, by the
+// smallest estimated time.  With the rows spread evenly (the counts are on the
+// device) an expert has mean +- sqrt(mean) of them, so its row tiles are one
+// while mean + 1.5 sqrt(mean) rows fit, else about mean / bm + 1/2.  A round of
+// tiles over the CUs takes the tile's operand bytes at the 20 B/clk a CU draws
+// from L2 plus ~2 us; in units of 128 bytes (2.67 ns) that is ks (bm + bn) +
+// 750.  No shape is faster than streaming the touched experts' weights (5.5
+// TB/s at best; few-rows tiles reach 1.15 times that time, the 256 x 256 ones
+// 1.4).  Between shapes at that floor, 128 columns are best for long K (32
+// steps and more) and 256 for short.  Measured (old = 256 x 256), us:
+//   gate/up 64 experts, D 2048, F 1024: 1 token, top-8, old 47.2, 32 x 64 19.0;
+//     48 tokens 148.9, 32 x 128 114.9; 768 tokens 146.5, 128 x 128 128.3;
+//   down, same layer: 27.3 -> 10.9, 58.3 -> 42.4, 68.7 -> 57.2;
+//   80 experts, D 1536, F 768: 333 tokens 98.7 -> 73.2 (64 x 256), 2048 tokens
+//     (205 rows each) 115.0, best other 132.1 (128 x 256): old;
+//   one segment, D 1536, F 768: 333 rows 35.9 -> 13.2 (64 x 64), 4096 rows
+//     39.6 -> 31.3 (128 x 256); 16384 rows, D 2048, F 1024 121.5 against 144.7;
+//   e4m3, 32 experts, D 4096, F 2048, top-4: 100 tokens 142.8 -> 115.3 and 56.5
+//     -> 42.7; 1600 tokens 159.9 against 172.9: old.
+void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int cus, int* bm, int* bn) {
+  const double n_eff = rows < n_experts ? static_cast<double>(rows) : n_experts;
+  const double mean = rows / n_eff;
+  const double ks = row_bytes / 128.0;
+  const double floor = n_eff * ncols * ks / (5.5e6 / 128.0) / 0.002667;
+  static const int kShapes[][2] = {{256, 256}, {128, 256}, {128, 128}, {64, 256}, {64, 128},
+                                   {64, 64},   {32, 256},  {32, 128},  {32, 64}};
+  double best = 0.0;
+  for (const auto& sh : kShapes) {
+    const bool old = sh[0] == 256;
+    double mt;
+    if (n_experts == 1)
+      mt = std::ceil(mean / sh[0]);
+    else
+      mt = n_eff * (mean + 1.5 * std::sqrt(mean) <= sh[0] ? 1.0 : mean / sh[0] + 0.5);
+    double cost = std::ceil(mt * (ncols / sh[1]) / cus) * (ks * (sh[0] + sh[1]) + 750.0);
+    double least = floor * (old ? 1.4 : 1.15);
+    if (!old) {
+      // shapes at the floor differ by little: weights read again for a second
+      // row tile, padding rows, and the width
+      least *= 1.0 + 0.15 * (mt / n_eff - 1.0) + 0.0004 * sh[0] +
+               (sh[1] == 64 ? 0.2 : (sh[1] == 128) == (ks >= 32.0) ? 0.0 : 0.01);
+    }
+    if (n_experts > 1 && cost < least) cost = least;
+    if (best == 0.0 || cost < best) {
+      best = cost;
+      *bm = sh[0];
+      *bn = sh[1];
+    }
+  }
+}
+
+// One tile shape of the few-rows kernel.
+template <int ELEM, int EPI, bool GATHER, int BM, int BN>
+int launch_few_tile(int grid, int dev, hipStream_t s, const uint8_t* a, const uint8_t* b,
+                    const float* a_scale, const float* b_scale, const int32_t* offsets,
+                    int n_experts, int kdim, int ncols, uint16_t* c, int64_t ldc,
+                    const int32_t* gather_src, int gather_k, int gather_rows, const uint16_t* dh,
+                    uint8_t* mx_exp) {
+  constexpr int kLds = FewCfg<ELEM, BM, BN>::kLds;
+  static std::atomic<uint64_t> done{0};  // devices whose LDS limit is set
+  const uint64_t bit = dev >= 0 && dev < 64 ? uint64_t(1) << dev : 0;
+  if (bit == 0 || (done.load(std::memory_order_acquire) & bit) == 0) {
+    if (!set_lds_limit(reinterpret_cast<const void*>(grouped_gemm_few<ELEM, EPI, GATHER, BM, BN>), kLds)) {
+      set_error("grouped GEMM: cannot allow %d bytes of dynamic LDS on device %d", kLds, dev);
+      return HMOE_ERR_HIP;
+    }
+    done.fetch_or(bit, std::memory_order_release);
+  }
+  hipLaunchKernelGGL((grouped_gemm_few<ELEM, EPI, GATHER, BM, BN>), dim3(grid), dim3(kThreads), kLds, s,
+                     a, b, a_scale, b_scale, offsets, n_experts, kdim, ncols, c, ldc, gather_src,
+                     gather_k, gather_rows, dh, mx_exp);
+  return HMOE_OK;
+}
+
+template <int ELEM, int EPI, bool GATHER, typename... Args>
+int launch_few(int bm, int bn, Args... args) {
+  if (bm == 32 && bn == 64) return launch_few_tile<ELEM, EPI, GATHER, 32, 64>(args...);
+  if (bm == 32 && bn == 128) return launch_few_tile<ELEM, EPI, GATHER, 32, 128>(args...);
+  if (bm == 32) return launch_few_tile<ELEM, EPI, GATHER, 32, 256>(args...);
+  if (bm == 64 && bn == 64) return launch_few_tile<ELEM, EPI, GATHER, 64, 64>(args...);
+  if (bm == 64 && bn == 128) return launch_few_tile<ELEM, EPI, GATHER, 64, 128>(args...);
+  if (bm == 64) return launch_few_tile<ELEM, EPI, GATHER, 64, 256>(args...);
+  if (bn == 128) return launch_few_tile<ELEM, EPI, GATHER, 128, 128>(args...);
+  return launch_few_tile<ELEM, EPI, GATHER, 128, 256>(args...);
+}
+
 int launch_grouped(bool swiglu, bool fp8, const void* A, const void* B, const float* a_scale,
                    const float* b_scale, const int32_t* offsets, int n_experts, int64_t rows_cap,
                    int kdim, int ncols, void* C, int64_t ldc, hipStream_t s, const char* what,
@@ -1983,6 +2541,34 @@ int launch_grouped(bool swiglu, bool fp8, const void* A, const void* B, const fl
   const uint8_t* b = static_cast<const uint8_t*>(B);
   uint16_t* c = static_cast<uint16_t*>(C);
   const bool odd = ((static_cast<int64_t>(kdim) * (fp8 ? 1 : 2) / 128) & 1) != 0;
+  int bm = 0, bn = 0;
+  choose_tile(rows_cap, n_experts, static_cast<int64_t>(kdim) * (fp8 ? 1 : 2), ncols, grid, &bm, &bn);
+  if (bm != kBM && (!fp8 || kdim % 128 == 0)) {
+#define HMOE_LAUNCH_FEW(EL, EP, GA)                                                             \
+  rc = launch_few<EL, EP, GA>(bm, bn, grid, dev, s, a, b, a_scale, b_scale, offsets, n_experts, kdim, \
+                              ncols, c, ldc, gather_src, gather_k, gather_rows, dswiglu_dh, mx_exp)
+    int rc = HMOE_OK;
+    const bool ga = gather_src != nullptr;
+    if (fp8) {
+      if (mx_exp != nullptr && swiglu && ga) HMOE_LAUNCH_FEW(kFewE4m3, kFewSwigluQ, true);
+      else if (mx_exp != nullptr && swiglu) HMOE_LAUNCH_FEW(kFewE4m3, kFewSwigluQ, false);
+      else if (mx_exp != nullptr) HMOE_LAUNCH_FEW(kFewE4m3Mx, kFewPlain, false);
+      else if (swiglu && ga) HMOE_LAUNCH_FEW(kFewE4m3, kFewSwiglu, true);
+      else if (swiglu) HMOE_LAUNCH_FEW(kFewE4m3, kFewSwiglu, false);
+      else HMOE_LAUNCH_FEW(kFewE4m3, kFewPlain, false);
+    } else if (dswiglu_dh != nullptr) {
+      if (ga) HMOE_LAUNCH_FEW(kFewBf16, kFewDSwiglu, true);
+      else HMOE_LAUNCH_FEW(kFewBf16, kFewDSwiglu, false);
+    } else if (swiglu) {
+      if (ga) HMOE_LAUNCH_FEW(kFewBf16, kFewSwiglu, true);
+      else HMOE_LAUNCH_FEW(kFewBf16, kFewSwiglu, false);
+    } else {
+      if (ga) HMOE_LAUNCH_FEW(kFewBf16, kFewPlain, true);
+      else HMOE_LAUNCH_FEW(kFewBf16, kFewPlain, false);
+    }
+#undef HMOE_LAUNCH_FEW
+    return rc != HMOE_OK ? rc : check_launch(what);
+  }
   if (fp8) {
     HMOE_REQUIRE(kdim % (2 * kW8StepBytes) == 0,
                  "%s: reduction dimension must be a multiple of %d", what, 2 * kW8StepBytes);
