@@ -1,11 +1,11 @@
 // Router aux outputs (model/moe.py:253-292): router_z_loss, balance_loss,
 // mean_entropy and expert_counts, from the router logits and top-k indices.
 //
-// Pass 1: one workgroup per 64-token chunk of one sequence; each wave takes
-// every fourth token, lanes own experts.  Per token it forms logsumexp,
+// Pass 1: one workgroup per 64-token chunk of one sequence; each of its 16
+// waves takes every sixteenth token, lanes own experts.  Per token it forms logsumexp,
 // sigmoid scores, the normalised routing distribution p and its entropy; it
-// accumulates p per expert and lse^2 / entropy per wave, then the four waves
-// are summed in a fixed order.  The chunk's per-sequence expert histogram is
+// accumulates p per expert and lse^2 / entropy per wave, then the waves are
+// summed in a fixed order.  The chunk's per-sequence expert histogram is
 // counted in LDS.  Pass 2: one workgroup reduces the chunk partials into the
 // four outputs.  Every float reduction has a fixed order, so results are
 // identical from run to run.
@@ -17,29 +17,42 @@ namespace {
 constexpr int kChunk = 64;
 constexpr int kMaxN = 256;
 
+// v plus the value of the lane the DPP control CTRL names (0 in the rows
+// ROW_MASK leaves out).
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+// Wave-wide sum, returned in every lane, on the VALU (the stages of
+// wave_max_f32): a shuffle through the LDS costs its latency per stage.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v = dpp_add<0xB1>(v);
+  v = dpp_add<0x4E>(v);
+  v = dpp_add<0x141>(v);
+  v = dpp_add<0x140>(v);
+  v = dpp_add<0x142, 0xA>(v);
+  v = dpp_add<0x143, 0xC>(v);
+  return lane_bcast(v, 63);
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
+__device__ __forceinline__ float wave_max(float v) { return wave_max_f32(v); }
 
 // Partial layout per chunk: probs[N], counts[N] (as int), z, ent.
 __host__ __device__ inline int64_t part_stride(int n) { return 2 * static_cast<int64_t>(n) + 2; }
 
+// 16 waves take 4 tokens of the chunk each, side by side, so that a chunk is
+// one token's chain of transcendentals and wave sums long and not sixteen
+// (bound by latency: 80 experts 27 us with four waves of 16 tokens in turn and
+// shuffles through the LDS).
+constexpr int kChunkWaves = 16;
+constexpr int kChunkTok = kChunk / kChunkWaves;
+
 template <int EPL>
-__global__ __launch_bounds__(256) void aux_chunk_kernel(const float* __restrict__ logits,
-                                                        const int32_t* __restrict__ top_idx,
-                                                        int seq, int n_experts, int top_k,
-                                                        int chunks_per_seq,
-                                                        float* __restrict__ parts) {
-  __shared__ float wprobs[4][kMaxN];
-  __shared__ float wz[4], went[4];
-  __shared__ int32_t hist[kMaxN];
+__global__ __launch_bounds__(64 * kChunkWaves) void aux_chunk_kernel(
+    const float* __restrict__ logits, const int32_t* __restrict__ top_idx, int seq, int n_experts,
+    int top_k, int chunks_per_seq, float* __restrict__ parts) {
+  __shared__ float wprobs[kChunkWaves][64 * EPL];
+  __shared__ float wz[kChunkWaves], went[kChunkWaves];
+  __shared__ int32_t hist[64 * EPL];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int chunk = blockIdx.x;
   const int b = chunk / chunks_per_seq;
@@ -47,9 +60,23 @@ __global__ __launch_bounds__(256) void aux_chunk_kernel(const float* __restrict_
   const int s0 = c * kChunk;
   const int s1 = min(seq, s0 + kChunk);
   const int64_t tok0 = static_cast<int64_t>(b) * seq;
-  for (int e = tid; e < n_experts; e += 256) hist[e] = 0;
+  // this wave's tokens s0 + wave + 16 q, loaded before anything waits
+  float l[kChunkTok][EPL];
+  bool live[kChunkTok];
+#pragma unroll
+  for (int q = 0; q < kChunkTok; ++q) {
+    const int s = s0 + wave + kChunkWaves * q;
+    live[q] = s < s1;  // uniform per wave
+    const float* row = logits + (tok0 + (live[q] ? s : s0)) * n_experts;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+      const int e = lane + 64 * j;
+      l[q][j] = row[e < n_experts ? e : n_experts - 1];
+    }
+  }
+  for (int e = tid; e < n_experts; e += 64 * kChunkWaves) hist[e] = 0;
   __syncthreads();
-  for (int i = tid; i < (s1 - s0) * top_k; i += 256) {
+  for (int i = tid; i < (s1 - s0) * top_k; i += 64 * kChunkWaves) {
     const int e = top_idx[(tok0 + s0) * top_k + i];
     if (static_cast<unsigned>(e) < static_cast<unsigned>(n_experts)) atomicAdd(&hist[e], 1);
   }
@@ -57,58 +84,73 @@ __global__ __launch_bounds__(256) void aux_chunk_kernel(const float* __restrict_
 #pragma unroll
   for (int j = 0; j < EPL; ++j) pacc[j] = 0.0f;
   float zacc = 0.0f, eacc = 0.0f;
-  for (int s = s0 + wave; s < s1; s += 4) {
-    const float* row = logits + (tok0 + s) * n_experts;
-    float l[EPL], sg[EPL];
-    float m = -__builtin_inff();
+  float m[kChunkTok], se[kChunkTok], ss[kChunkTok], ent[kChunkTok];
+#pragma unroll
+  for (int q = 0; q < kChunkTok; ++q) {
+    m[q] = -__builtin_inff();
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
-      const int e = lane + 64 * j;
-      l[j] = e < n_experts ? row[e] : -__builtin_inff();
-      m = fmaxf(m, l[j]);
+      if (lane + 64 * j >= n_experts) l[q][j] = -__builtin_inff();
+      m[q] = fmaxf(m[q], l[q][j]);
     }
-    m = wave_max(m);
-    float se = 0.0f, ss = 0.0f;
+    m[q] = wave_max(m[q]);
+  }
+  float sg[kChunkTok][EPL];
+#pragma unroll
+  for (int q = 0; q < kChunkTok; ++q) {
+    se[q] = 0.0f;
+    ss[q] = 0.0f;
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
       const bool ok = lane + 64 * j < n_experts;
-      se += ok ? expf(l[j] - m) : 0.0f;
-      sg[j] = ok ? sigmoid_det(l[j]) : 0.0f;
-      ss += sg[j];
+      se[q] += ok ? expf(l[q][j] - m[q]) : 0.0f;
+      sg[q][j] = ok ? sigmoid_det(l[q][j]) : 0.0f;
+      ss[q] += sg[q][j];
     }
-    se = wave_sum(se);
-    ss = wave_sum(ss);
-    const float lse = m + logf(se);
-    float ent = 0.0f;
-    const float inv = 1.0f / (ss + 1e-9f);
+    se[q] = wave_sum(se[q]);
+    ss[q] = wave_sum(ss[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < kChunkTok; ++q) {
+    ent[q] = 0.0f;
+    const float inv = 1.0f / (ss[q] + 1e-9f);
 #pragma unroll
     for (int j = 0; j < EPL; ++j) {
-      const float p = sg[j] * inv;
-      pacc[j] += p;
-      if (lane + 64 * j < n_experts) ent -= p * logf(p + 1e-9f);
+      const float p = sg[q][j] * inv;
+      if (live[q]) pacc[j] += p;
+      if (lane + 64 * j < n_experts) ent[q] -= p * logf(p + 1e-9f);
     }
-    ent = wave_sum(ent);
-    zacc += lse * lse;
-    eacc += ent;
+    ent[q] = wave_sum(ent[q]);
+    const float lse = m[q] + logf(se[q]);
+    if (live[q]) {
+      zacc += lse * lse;
+      eacc += ent[q];
+    }
   }
 #pragma unroll
-  for (int j = 0; j < EPL; ++j) {
-    const int e = lane + 64 * j;
-    if (e < n_experts) wprobs[wave][e] = pacc[j];
-  }
+  for (int j = 0; j < EPL; ++j) wprobs[wave][lane + 64 * j] = pacc[j];
   if (lane == 0) {
     wz[wave] = zacc;
     went[wave] = eacc;
   }
   __syncthreads();
   float* out = parts + static_cast<int64_t>(chunk) * part_stride(n_experts);
-  for (int e = tid; e < n_experts; e += 256) {
-    out[e] = ((wprobs[0][e] + wprobs[1][e]) + wprobs[2][e]) + wprobs[3][e];
+  for (int e = tid; e < n_experts; e += 64 * kChunkWaves) {
+    float p = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kChunkWaves; ++w) p += wprobs[w][e];
+    out[e] = p;
     reinterpret_cast<int32_t*>(out)[n_experts + e] = hist[e];
   }
   if (tid == 0) {
-    out[2 * n_experts] = ((wz[0] + wz[1]) + wz[2]) + wz[3];
-    out[2 * n_experts + 1] = ((went[0] + went[1]) + went[2]) + went[3];
+    float z = 0.0f, en = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kChunkWaves; ++w) {
+      z += wz[w];
+      en += went[w];
+    }
+    out[2 * n_experts] = z;
+    out[2 * n_experts + 1] = en;
   }
 }
 
@@ -342,11 +384,11 @@ extern "C" int hmoe_router_aux(const float* logits, const int32_t* top_idx, int 
   const dim3 grid(static_cast<unsigned>(batch * cps));
   float* parts = static_cast<float*>(workspace);
   if (n_experts <= 64)
-    hipLaunchKernelGGL(aux_chunk_kernel<1>, grid, dim3(256), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
+    hipLaunchKernelGGL(aux_chunk_kernel<1>, grid, dim3(64 * kChunkWaves), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
   else if (n_experts <= 128)
-    hipLaunchKernelGGL(aux_chunk_kernel<2>, grid, dim3(256), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
+    hipLaunchKernelGGL(aux_chunk_kernel<2>, grid, dim3(64 * kChunkWaves), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
   else
-    hipLaunchKernelGGL(aux_chunk_kernel<4>, grid, dim3(256), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
+    hipLaunchKernelGGL(aux_chunk_kernel<4>, grid, dim3(64 * kChunkWaves), 0, s, logits, top_idx, seq, n_experts, top_k, cps, parts);
   if (int rc = check_launch("router_aux/chunk")) return rc;
   hipLaunchKernelGGL(aux_final_kernel, dim3(1), dim3(kFinalThreads), 0, s, parts, batch, seq,
                      n_experts, top_k, cps, losses, expert_counts);

@@ -312,6 +312,12 @@ constexpr int kFusedScanBlocks = 256;
 // 1024 experts (65536 entries) 22.6 against 22.4 us.
 constexpr int64_t kFusedScanEntries = 65536;
 
+// SELF: plans of at most kSelfHistRows slots count the whole top_idx in every
+// workgroup instead (8 loads in flight a thread, LDS atomics on exact integers),
+// so the plan is one launch.
+constexpr int64_t kSelfHistRows = 8192;
+
+template <bool SELF>
 __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
     const int32_t* __restrict__ top_idx, int64_t rows, int n_experts, int64_t capacity,
     const int32_t* __restrict__ hist, int nblk, int32_t* __restrict__ counts,
@@ -347,30 +353,55 @@ __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
   // tid taking experts tid, tid + 256, ... when N > 256); group g sums the
   // blocks g, g + G, ..., so the 64 lanes of a wave read 64 consecutive
   // experts of one block.
-  const int G = n_experts >= kPlanThreads ? 1 : kPlanThreads / n_experts;
-  for (int idx = tid; idx < (G > 1 ? G * n_experts : n_experts); idx += kPlanThreads) {
-    const int g = G > 1 ? idx / n_experts : 0;
-    const int e = G > 1 ? idx - g * n_experts : idx;
-    int32_t pre = 0, tot = 0;
-    int bb = g;
-    // eight loads in flight at a time (the sums are exact integer sums)
-    for (; bb + 7 * G < nblk; bb += 8 * G) {
-      int32_t c[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) c[u] = hist[static_cast<int64_t>(bb + u * G) * n_experts + e];
+  const int G = SELF || n_experts >= kPlanThreads ? 1 : kPlanThreads / n_experts;
+  if constexpr (SELF) {
+    for (int e = tid; e < n_experts; e += kPlanThreads) {
+      part_pre[e] = 0;
+      part_tot[e] = 0;
+    }
+    __syncthreads();
+    const int n = static_cast<int>(rows), before = static_cast<int>(blk_base);
+    for (int i0 = tid; i0 < n; i0 += 8 * kPlanThreads) {
+      int v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        tot += c[u];
-        if (bb + u * G < b) pre += c[u];
+        const int i = i0 + u * kPlanThreads;
+        v[u] = top_idx[i < n ? i : n - 1];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int i = i0 + u * kPlanThreads;
+        if (i < n && static_cast<unsigned>(v[u]) < static_cast<unsigned>(n_experts)) {
+          atomicAdd(&part_tot[v[u]], 1);
+          if (i < before) atomicAdd(&part_pre[v[u]], 1);
+        }
       }
     }
-    for (; bb < nblk; bb += G) {
-      const int32_t c = hist[static_cast<int64_t>(bb) * n_experts + e];
-      tot += c;
-      if (bb < b) pre += c;
+  } else {
+    for (int idx = tid; idx < (G > 1 ? G * n_experts : n_experts); idx += kPlanThreads) {
+      const int g = G > 1 ? idx / n_experts : 0;
+      const int e = G > 1 ? idx - g * n_experts : idx;
+      int32_t pre = 0, tot = 0;
+      int bb = g;
+      // eight loads in flight at a time (the sums are exact integer sums)
+      for (; bb + 7 * G < nblk; bb += 8 * G) {
+        int32_t c[8];
+  #pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = hist[static_cast<int64_t>(bb + u * G) * n_experts + e];
+  #pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          tot += c[u];
+          if (bb + u * G < b) pre += c[u];
+        }
+      }
+      for (; bb < nblk; bb += G) {
+        const int32_t c = hist[static_cast<int64_t>(bb) * n_experts + e];
+        tot += c;
+        if (bb < b) pre += c;
+      }
+      part_pre[idx] = pre;
+      part_tot[idx] = tot;
     }
-    part_pre[idx] = pre;
-    part_tot[idx] = tot;
   }
   __syncthreads();
   // Per expert: base of this block, total, kept rows (in part_tot[e]).
@@ -659,12 +690,19 @@ int launch_plan(const int32_t* top_idx, int64_t tokens, int top_k, int n_experts
   const int64_t rows = tokens * top_k;
   const int64_t rows_cap = hmoe_rows_cap(tokens, top_k, n_experts, capacity);
   const int nblk = static_cast<int>(plan_blocks(rows));
+  // (few experts' counters in one workgroup serialise its atomics: from 8 up)
+  if (rows > 0 && (rows <= kSlotsPerBlock || (rows <= kSelfHistRows && n_experts >= 8))) {
+    hipLaunchKernelGGL(plan_rank_fused_kernel<true>, dim3(nblk), dim3(kPlanThreads), 0, s, top_idx,
+                       rows, n_experts, capacity, static_cast<const int32_t*>(nullptr), nblk, counts,
+                       offsets, slot_pos, perm_src, keep, rows_cap);
+    return check_launch("dispatch_plan/rank");
+  }
   if (rows > 0 && nblk <= kFusedScanBlocks &&
       static_cast<int64_t>(nblk) * n_experts <= kFusedScanEntries) {
     hipLaunchKernelGGL(plan_histogram_kernel, dim3(nblk), dim3(kPlanThreads), 0, s, top_idx, rows,
                        n_experts, hist);
     if (int rc = check_launch("dispatch_plan/histogram")) return rc;
-    hipLaunchKernelGGL(plan_rank_fused_kernel, dim3(nblk), dim3(kPlanThreads), 0, s, top_idx, rows,
+    hipLaunchKernelGGL(plan_rank_fused_kernel<false>, dim3(nblk), dim3(kPlanThreads), 0, s, top_idx, rows,
                        n_experts, capacity, hist, nblk, counts, offsets, slot_pos, perm_src, keep,
                        rows_cap);
     return check_launch("dispatch_plan/rank");
