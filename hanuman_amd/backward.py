@@ -125,7 +125,7 @@ def shared_backward(xc: torch.Tensor, d_shared: torch.Tensor, h_shared, ops: Sha
     float32 sum for several) and ``dWg``, ``dWu``, ``dWd`` in the parameter
     shapes."""
     T = xc.shape[0]
-    off = torch.tensor([0, T], dtype=torch.int32, device=xc.device)
+    off = K.one_group_offsets(T, xc.device)
     dxs, dwg, dwu, dwd = [], [], [], []
     for (fwd_gu, gu_dgrad, down_dgrad), h in zip(ops.experts, h_shared):
         dh = K.grouped_dgrad_down(d_shared, off, down_dgrad)
@@ -234,7 +234,7 @@ def _shared_backward_f32(x32: torch.Tensor, d_shared: torch.Tensor, h_shared, ma
     if n_shared == 1:
         w_gate, w_up, w_down = (w.unsqueeze(0) for w in (w_gate, w_up, w_down))
     T = x32.shape[0]
-    off = torch.tensor([0, T], dtype=torch.int32, device=x32.device)
+    off = K.one_group_offsets(T, x32.device)
     dx, dwg, dwu, dwd = None, [], [], []
     for i, h in enumerate(h_shared):
         wg, wu, wd = (w[i:i + 1].contiguous() for w in (w_gate, w_up, w_down))

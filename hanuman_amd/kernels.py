@@ -171,6 +171,15 @@ def dispatch_plan(top_idx: torch.Tensor, n_experts: int, cap: int,
     return Plan(counts, offsets, slot_pos, perm_src, keep, cap, rc, n_experts, K)
 
 
+def one_group_offsets(rows: int, device) -> torch.Tensor:
+    """Segment offsets ``[0, rows]`` of one group, made on the device: a tensor
+    from a host list is a copy that the host waits for, and with it for
+    everything enqueued before."""
+    if rows == 0:
+        return torch.zeros(2, dtype=torch.int32, device=device)
+    return torch.arange(0, 2 * rows, rows, dtype=torch.int32, device=device)
+
+
 def permute_rows(x: torch.Tensor, plan: Plan, out_dtype: torch.dtype = torch.bfloat16):
     """Dispatched rows ``xs [rows_cap, D]`` (``moe.py:56,198``); token-centric."""
     _check(x, "x", 2)

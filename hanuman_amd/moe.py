@@ -72,7 +72,7 @@ def _f32_swiglu_one(x32: torch.Tensor, wg, wu, wd, hs: list | None = None) -> to
     """One float32 SwiGLU (``moe.py:23-29`` with dtype float32): one segment
     of all rows on the float32 grouped GEMMs, masters as they are.  ``hs``
     collects ``h`` for the backward."""
-    off = _offsets_one_group(x32.shape[0], x32.device)
+    off = K.one_group_offsets(x32.shape[0], x32.device)
     h = K.grouped_gate_up_f32(x32, off, wg.float().unsqueeze(0).contiguous(),
                               wu.float().unsqueeze(0).contiguous())
     if hs is not None:
@@ -109,10 +109,6 @@ class _PackCache:
         return self._val
 
 
-def _offsets_one_group(rows: int, device) -> torch.Tensor:
-    return torch.tensor([0, rows], dtype=torch.int32, device=device)
-
-
 def swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
            dtype) -> torch.Tensor:
     """Dense SwiGLU ``down(silu(x@gate) * (x@up))`` -> float32 (``moe.py:23-29``).
@@ -127,7 +123,7 @@ def swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: to
         return _f32_swiglu_one(x.float().contiguous(), w_gate, w_up, w_down)
     xb = x.to(dt).contiguous()
     T = xb.shape[0]
-    off = _offsets_one_group(T, x.device)
+    off = K.one_group_offsets(T, x.device)
     wgu = K.pack_gate_up(w_gate.unsqueeze(0).contiguous(), w_up.unsqueeze(0).contiguous())
     wd = K.pack_down(w_down.unsqueeze(0).contiguous())
     h = K.grouped_gate_up(xb, off, wgu)
@@ -291,7 +287,7 @@ class MoE:
         if self.n_shared_experts == 0:
             return 0.0 / self.n_shared_experts  # ZeroDivisionError, as the reference
         T = x_flat.shape[0]
-        off = _offsets_one_group(T, x_flat.device)
+        off = K.one_group_offsets(T, x_flat.device)
         outs = []
         if self.dtype == torch.float32:
             wg, wu, wdn = self.shared_w_gate.value, self.shared_w_up.value, self.shared_w_down.value
