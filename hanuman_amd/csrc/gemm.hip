@@ -1692,7 +1692,7 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
 // rounded up to even, with no masking, and no buffer size limits it.  The output is float32; SPLIT: B's
 // columns are in the gate/up order (blocks of 32 gate columns, then the 32 up
 // columns of the same h columns) and C goes to out0 (gate) and out1 (up) as
-// [e][m][F].
+// [e][m][F].  Few rows an expert make the gradient stores the bound.
 template <bool SPLIT, bool BIG>
 __global__ __launch_bounds__(kThreads) void grouped_gemm_wgrad(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
@@ -1908,30 +1908,45 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_wgrad(
       if (kb + 2 < ct.kpad) read_frags(0, 0, 0);
     }
     // Epilogue: acc[i][j] lane L element r is C[m][n] with m = wm*128 + 32i +
-    // L%32, n = wn*128 + 32j + (r/4)*8 + (L/32)*4 + r%4 (tile-relative).
+    // L%32, n = wn*128 + 32j + (r/4)*8 + (L/32)*4 + r%4 (tile-relative).  The
+    // float32 tile leaves through the idle stage 1 in four passes of 64 rows
+    // (rows i of every wave, 1024 bytes each, 16-byte chunk c of row l at c ^
+    // (l & 31)), so that a wave's store is one whole row: 1 KB, or 512 bytes of
+    // the gate's and of the up's gradient.  Stored straight from the
+    // accumulators, 16 bytes of each of 32 rows an instruction, the stores of
+    // 205 rows an expert's gradients ran at 1.7 TB/s.
     const int frow = lane & 31;
-    const int col_lane = (lane >> 5) * 4;
+    const int half = lane >> 5;
     const int F = N / 2;
+    uint8_t* const st = smem + kStageBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int64_t m = ct.m0 + wm * 128 + 32 * i + frow;
+      const int l = wm * 32 + frow;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const int n = ct.n0 + wn * 128 + 32 * j + g * 8 + col_lane;
           const f32x4 v = {acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2],
                            acc[i][j][g * 4 + 3]};
-          float* dst;
-          if (SPLIT) {
-            const int f = (n >> 6) * 32 + (n & 31);
-            dst = ((n & 63) < 32 ? out0 : out1) + (static_cast<int64_t>(ct.e) * M + m) * F + f;
-          } else {
-            dst = out0 + (static_cast<int64_t>(ct.e) * M + m) * N + n;
-          }
-          __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(dst));
+          const int c = wn * 32 + j * 8 + g * 2 + half;
+          *reinterpret_cast<f32x4*>(st + l * 1024 + ((c ^ (l & 31)) * 16)) = v;
         }
       __builtin_amdgcn_sched_barrier(0);
+      barrier_lds();
+      // wave w stores rows w, w + 4, ... of the pass, lane c chunk c
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int r = wave + 4 * q;  // LDS row: tile row (r / 32) * 128 + 32 i + r % 32
+        const f32x4 v = *reinterpret_cast<const f32x4*>(st + r * 1024 + ((lane ^ (r & 31)) * 16));
+        const int64_t row = static_cast<int64_t>(ct.e) * M + ct.m0 + (r >> 5) * 128 + 32 * i + (r & 31);
+        float* dst;
+        if (SPLIT)
+          dst = ((lane & 8) ? out1 : out0) + row * F + ct.n0 / 2 + (lane >> 4) * 32 + (lane & 7) * 4;
+        else
+          dst = out0 + row * N + ct.n0 + lane * 4;
+        __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(dst));
+      }
+      barrier_lds();
     }
   }
 }
