@@ -35,6 +35,9 @@
 // the segment's rows 16 at a time (rows past it load as zero; an empty
 // segment writes zeros).  Columns at or past nsplit go to a second output
 // (dWu beside dWg).
+#include <algorithm>
+#include <atomic>
+
 #include "hmoe_common.h"
 
 namespace hmoe {
@@ -283,6 +286,300 @@ __global__ __launch_bounds__(256) void grouped_wgrad_f32_kernel(
   }
 }
 
+// ---- few tiles: K split over the waves ----------------------------------------
+// Where 64 x 64 tiles are fewer than the CUs (a short prompt, one shared expert,
+// a weight gradient of few experts), the kernels above are bound by the latency
+// of their K steps.  Here a workgroup's 4 waves share one 32 x 32 tile and split
+// K: wave w takes the 32-long K chunks w, w + 4, ..., its operands going from
+// global memory straight into registers in the MFMA's layout, a chunk (16
+// MFMAs) ahead, with no LDS and no barrier in the loop; the four partial tiles
+// are added through LDS in wave order and each wave finishes a quarter of the
+// columns.  An MFMA sums k and k + 4 of a chunk's groups of 8 (any order serves
+// both operands alike), so a row-major A is read 16 bytes a lane; the waves'
+// chunks of a row share its lines.  Four times the tiles and four waves in K:
+// 16 times the chains.  Measured, us (64 x 64 -> split; d_model 256, d_ff 512):
+// one 2048-row segment, down 18.3 -> 13.2 (128 tiles), its weight gradients 62.4
+// -> 14.6 and 63.4 -> 16.4 (32, 64 tiles); 80 rows on 8 experts, gate/up 16.3 ->
+// 7.6, down 17.8 -> 7.3; 8 experts' weight gradients over 4096 rows 26.3 -> 18.3
+// (256 tiles) and 32.2 -> 27.8 (512).  Past the lines below the operands' traffic
+// (twice that of a 64 x 64 tile) loses: gate/up of 2048 rows 17.1 against 22.4
+// (256 tiles), 16 experts' weight gradients (1536 tiles) 30.2 against 38.8.
+constexpr int kF32Split = 32;
+
+// A lane's f32x4 groups of the four waves' partial fragments, added in wave
+// order: part[wave][fragment][q][lane].
+__device__ __forceinline__ f32x4 sum_parts(const f32x4* part, int frags, int f, int q, int lane) {
+  f32x4 v = part[(f * 4 + q) * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    const f32x4 t = part[((w * frags + f) * 4 + q) * 64 + lane];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] += t[r];
+  }
+  return v;
+}
+
+template <int EPI, bool BT>
+__global__ __launch_bounds__(256) void grouped_gemm_f32_split_kernel(
+    const float* __restrict__ A, const float* __restrict__ B0, const float* __restrict__ B1,
+    const int32_t* __restrict__ offsets, int n_experts, int kdim, int ksplit, int ncols,
+    const float* __restrict__ dh, float* __restrict__ C, int64_t ldc) {
+  constexpr bool kDual = EPI != kEpiPlain;  // two accumulators (g and u)
+  constexpr int kMats = kDual ? 2 : 1;
+  __shared__ int32_t mstart[kF32MaxExperts + 1];
+  __shared__ int32_t scan[256];
+  __shared__ f32x4 part[4 * kMats * 4 * 64];
+  const int tid = threadIdx.x;
+  // per-expert row-tile starts (exclusive scan of ceil(rows_e / kF32Split))
+  const int per = (n_experts + 255) / 256;
+  int local = 0;
+  for (int j = 0; j < per; ++j) {
+    const int e = tid * per + j;
+    if (e < n_experts) local += (offsets[e + 1] - offsets[e] + kF32Split - 1) / kF32Split;
+  }
+  scan[tid] = local;
+  __syncthreads();
+  for (int off = 1; off < 256; off <<= 1) {
+    const int v = tid >= off ? scan[tid - off] : 0;
+    __syncthreads();
+    scan[tid] += v;
+    __syncthreads();
+  }
+  int run = scan[tid] - local;
+  for (int j = 0; j < per; ++j) {
+    const int e = tid * per + j;
+    if (e < n_experts) {
+      mstart[e] = run;
+      run += (offsets[e + 1] - offsets[e] + kF32Split - 1) / kF32Split;
+    }
+  }
+  if (tid == 255) mstart[n_experts] = scan[255];
+  __syncthreads();
+  const int n_tiles_n = ncols / kF32Split;
+  const int m_tile = blockIdx.x / n_tiles_n;
+  const int n0 = (blockIdx.x - m_tile * n_tiles_n) * kF32Split;
+  if (m_tile >= mstart[n_experts]) return;  // uniform per workgroup
+  int lo = 0, hi = n_experts;  // largest e with mstart[e] <= m_tile
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (mstart[mid] <= m_tile) lo = mid; else hi = mid;
+  }
+  const int e = __builtin_amdgcn_readfirstlane(lo);
+  const int64_t row0 = offsets[e] + static_cast<int64_t>(m_tile - mstart[e]) * kF32Split;
+  const int64_t row_end = offsets[e + 1];
+  // each B matrix is ksplit long along K; expert stride ksplit * ncols
+  const int64_t bstride = static_cast<int64_t>(ksplit) * ncols;
+  const float* be0 = B0 + e * bstride;
+  const float* be1 = B1 != nullptr ? B1 + e * bstride : be0;
+
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hi2 = lane >> 5;
+  // this lane's row (past the segment: its last one)
+  const float* arow = A + (row0 + l32 < row_end ? row0 + l32 : row_end - 1) * kdim;
+  const int n = n0 + l32;
+  // One chunk of 32 k: group g of 8 k, lane half hi2 holds k = 8 g + 4 hi2 + 0..3.
+  struct Chunk {
+    f32x4 a[4];
+    f32x4 b[kMats][4];
+  };
+  auto load = [&](Chunk& c, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int k = k0 + 8 * g + 4 * hi2;
+      c.a[g] = *reinterpret_cast<const f32x4*>(arow + k);
+#pragma unroll
+      for (int m = 0; m < kMats; ++m) {
+        // (a single matrix changes to the second one at ksplit, a multiple of 32)
+        const float* be = m == 1 || (!kDual && k0 >= ksplit) ? be1 : be0;
+        const int kb = !kDual && k0 >= ksplit ? k - ksplit : k;
+        f32x4& v = c.b[m][g];
+        if constexpr (BT) {
+          v = *reinterpret_cast<const f32x4*>(be + static_cast<int64_t>(n) * ksplit + kb);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = be[static_cast<int64_t>(kb + r) * ncols + n];
+        }
+      }
+    }
+  };
+  // The last 16 k of a K that is an odd multiple of 16 (a single matrix, or g
+  // and u: a two-phase K is a multiple of 128): zeros past it.
+  auto load_tail = [&](Chunk& c, int k0) __attribute__((always_inline)) {
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int k = k0 + 8 * g + 4 * hi2;
+      c.a[g] = g < 2 ? *reinterpret_cast<const f32x4*>(arow + k) : zero;
+#pragma unroll
+      for (int m = 0; m < kMats; ++m) {
+        const float* be = m == 1 ? be1 : be0;
+        f32x4 v = zero;
+        if (g < 2) {
+          if (BT) {
+            v = *reinterpret_cast<const f32x4*>(be + static_cast<int64_t>(n) * ksplit + k);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = be[static_cast<int64_t>(k + r) * ncols + n];
+          }
+        }
+        c.b[m][g] = v;
+      }
+    }
+  };
+  f32x16 acc[kMats];
+#pragma unroll
+  for (int m = 0; m < kMats; ++m)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[m][r] = 0.0f;
+  // D[n][m] += B^T[n][k] A^T[k][m]: the weights are the first operand, so that
+  // a lane ends with one token row and groups of 4 columns
+  auto compute = [&](const Chunk& c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int m = 0; m < kMats; ++m) acc[m] = mfma32x2(c.b[m][g][r], c.a[g][r], acc[m]);
+  };
+  const int nfull = kdim / 32;
+  Chunk c0, c1;
+  int ch = wave;
+  if (ch < nfull) load(c0, ch * 32);
+  for (; ch < nfull; ch += 8) {
+    if (ch + 4 < nfull) load(c1, (ch + 4) * 32);
+    compute(c0);
+    if (ch + 4 >= nfull) break;
+    if (ch + 8 < nfull) load(c0, (ch + 8) * 32);
+    compute(c1);
+  }
+  if (kdim % 32 != 0 && (nfull & 3) == wave) {
+    load_tail(c0, nfull * 32);
+    compute(c0);
+  }
+#pragma unroll
+  for (int m = 0; m < kMats; ++m)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      f32x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = acc[m][4 * q + r];
+      part[((wave * kMats + m) * 4 + q) * 64 + lane] = v;
+    }
+  __syncthreads();
+  // Wave w finishes group q = w: lane row l32, columns 8 w + 4 hi2 + 0..3.
+  const int64_t row = row0 + l32;
+  if (row >= row_end) return;
+  const int col = n0 + 8 * wave + 4 * hi2;
+  const f32x4 g4 = sum_parts(part, kMats, 0, wave, lane);
+  f32x4 v = g4;
+  if constexpr (kDual) {
+    const f32x4 u4 = sum_parts(part, kMats, 1, wave, lane);
+    if constexpr (EPI == kEpiSwiglu) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = (g4[r] / (1.0f + expf(-g4[r]))) * u4[r];
+    } else {
+#pragma clang fp contract(off)
+      const f32x4 d = *reinterpret_cast<const f32x4*>(dh + row * ncols + col);
+      f32x4 w;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float sg = 1.0f / (1.0f + expf(-g4[r]));
+        v[r] = d[r] * u4[r] * (sg * (1.0f + g4[r] * (1.0f - sg)));
+        w[r] = d[r] * (g4[r] * sg);
+      }
+      *reinterpret_cast<f32x4*>(C + row * ldc + ncols + col) = w;
+    }
+  }
+  *reinterpret_cast<f32x4*>(C + row * ldc + col) = v;
+}
+
+__global__ __launch_bounds__(256) void grouped_wgrad_f32_split_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
+    const int32_t* __restrict__ offsets, int mdim, int ncols, int nsplit, float* __restrict__ C0,
+    float* __restrict__ C1) {
+  __shared__ f32x4 part[4 * 4 * 64];
+  const int tid = threadIdx.x;
+  const int tm = mdim / kF32Split, tn = ncols / kF32Split;
+  const int e = static_cast<int>(blockIdx.x / (tm * tn));
+  const int rem = static_cast<int>(blockIdx.x - static_cast<int64_t>(e) * tm * tn);
+  const int m0 = (rem / tn) * kF32Split;
+  const int n0 = (rem - (rem / tn) * tn) * kF32Split;
+  const int64_t r_lo = __builtin_amdgcn_readfirstlane(offsets[e]);
+  const int rows = __builtin_amdgcn_readfirstlane(offsets[e + 1]) - static_cast<int>(r_lo);
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hi2 = lane >> 5;
+  // One chunk of 32 rows: MFMA s takes rows 2 s + hi2.  The resources start at
+  // the chunk and end at the segment, so later rows read as zeros.
+  struct Chunk {
+    float a[16];
+    float b[16];
+  };
+  const int a_voff = (hi2 * static_cast<int>(lda) + m0 + l32) * 4;
+  const int b_voff = (hi2 * static_cast<int>(ldb) + n0 + l32) * 4;
+  auto load = [&](Chunk& c, int r0) __attribute__((always_inline)) {
+    const int left = rows - r0 < 32 ? rows - r0 : 32;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(A + (r_lo + r0) * lda), 0, left * static_cast<int>(lda) * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(B + (r_lo + r0) * ldb), 0, left * static_cast<int>(ldb) * 4, 0x00020000);
+    // (the row offset is in the range-checked vector offset)
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      c.a[s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+          ra, a_voff + 2 * s * static_cast<int>(lda) * 4, 0, 0));
+      c.b[s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+          rb, b_voff + 2 * s * static_cast<int>(ldb) * 4, 0, 0));
+    }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  // D[n][m] += B^T[n][k] A[k][m], so that a lane ends with one output row m
+  auto compute = [&](const Chunk& c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) acc = mfma32x2(c.b[s], c.a[s], acc);
+  };
+  const int n_ch = (rows + 31) / 32;
+  Chunk c0, c1;
+  int ch = wave;
+  if (ch < n_ch) load(c0, ch * 32);
+  for (; ch < n_ch; ch += 8) {
+    if (ch + 4 < n_ch) load(c1, (ch + 4) * 32);
+    compute(c0);
+    if (ch + 4 >= n_ch) break;
+    if (ch + 8 < n_ch) load(c0, (ch + 8) * 32);
+    compute(c1);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = acc[4 * q + r];
+    part[(wave * 4 + q) * 64 + lane] = v;
+  }
+  __syncthreads();
+  // wave w finishes group q = w: row m0 + l32, columns 8 w + 4 hi2 + 0..3
+  const int64_t m = static_cast<int64_t>(e) * mdim + m0 + l32;
+  const f32x4 v = sum_parts(part, 1, 0, wave, lane);
+  const int col = n0 + 8 * wave + 4 * hi2;
+  float* dst = n0 < nsplit ? C0 + m * nsplit + col : C1 + m * (ncols - nsplit) + (col - nsplit);
+  *reinterpret_cast<f32x4*>(dst) = v;
+}
+
+// CUs of the stream's device (256 if it cannot be queried), cached per device.
+int f32_cus(hipStream_t s) {
+  int dev = 0;
+  if (hipStreamGetDevice(s, &dev) != hipSuccess && hipGetDevice(&dev) != hipSuccess) return 256;
+  static std::atomic<int> cached[64];
+  int cus = dev >= 0 && dev < 64 ? cached[dev].load(std::memory_order_relaxed) : 0;
+  if (cus == 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      return 256;
+    if (dev >= 0 && dev < 64) cached[dev].store(cus, std::memory_order_relaxed);
+  }
+  return cus;
+}
+
 template <int EPI, bool BT>
 int launch_f32(const float* A, const float* B0, const float* B1, const int32_t* offsets,
                int n_experts, int64_t rows_cap, int kdim, int ksplit, int ncols, const float* dh,
@@ -290,6 +587,14 @@ int launch_f32(const float* A, const float* B0, const float* B1, const int32_t* 
   const int64_t m_tiles = ceil_div(rows_cap, kF32Tile) + n_experts;
   const int64_t grid = m_tiles * (ncols / kF32Tile);
   HMOE_REQUIRE(grid < (int64_t(1) << 31), "%s: too many tiles", what);
+  // fewer 64 x 64 tiles than three quarters of the CUs (rows_cap rows at most)
+  if (ceil_div(rows_cap, kF32Tile) * (ncols / kF32Tile) * 4 < int64_t(3) * f32_cus(s)) {
+    const int64_t split = (ceil_div(rows_cap, kF32Split) + std::min<int64_t>(n_experts, rows_cap)) *
+                          (ncols / kF32Split);
+    hipLaunchKernelGGL((grouped_gemm_f32_split_kernel<EPI, BT>), dim3(static_cast<unsigned>(split)),
+                       dim3(256), 0, s, A, B0, B1, offsets, n_experts, kdim, ksplit, ncols, dh, C, ldc);
+    return check_launch(what);
+  }
   hipLaunchKernelGGL((grouped_gemm_f32_kernel<EPI, BT>), dim3(static_cast<unsigned>(grid)), dim3(256),
                      0, s, A, B0, B1, offsets, n_experts, kdim, ksplit, ncols, dh, C, ldc);
   return check_launch(what);
@@ -300,6 +605,11 @@ int launch_wgrad_f32(const float* A, int64_t lda, const float* B, int64_t ldb,
                      float* C0, float* C1, hipStream_t s, const char* what) {
   const int64_t grid = static_cast<int64_t>(n_experts) * (mdim / kF32Tile) * (ncols / kF32Tile);
   HMOE_REQUIRE(grid < (int64_t(1) << 31), "%s: too many tiles", what);
+  if (grid <= int64_t(2) * f32_cus(s)) {
+    hipLaunchKernelGGL(grouped_wgrad_f32_split_kernel, dim3(static_cast<unsigned>(4 * grid)), dim3(256),
+                       0, s, A, lda, B, ldb, offsets, mdim, ncols, nsplit, C0, C1);
+    return check_launch(what);
+  }
   hipLaunchKernelGGL(grouped_wgrad_f32_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, A,
                      lda, B, ldb, offsets, mdim, ncols, nsplit, C0, C1);
   return check_launch(what);
