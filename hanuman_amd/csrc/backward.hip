@@ -346,22 +346,12 @@ __global__ __launch_bounds__(256) void router_dx_kernel(const float* __restrict_
 
 // d_router[d, n] = sum_t x[t, d] * d_logits[t, n] (the VJP of x_f @ router,
 // moe.py:178, with respect to the router weight), float32, in two passes for
-// a fixed summation order: pass 1 sums chunks of tokens into
+// a fixed summation order: pass 1 sums chunks of kRdwChunk tokens into
 // partials [chunk][D][N]; pass 2 sums the chunks in order.  Pass 1
 // workgroup tile: 128 d x 64 n of one chunk; wave w owns d 32 w .. +32 and
 // both 32-column n blocks (A = x^T, B = d_logits); tokens staged 64 at a time
 // in LDS as [token][d] and [token][n].
-// Tokens per chunk: the most of 512, 256, 128, 64 that still give 256
-// workgroups (one per CU), else 64.  At 2048 tokens 512 left 8 workgroups for d_model
-// 256 / 8 experts and 96 for 1536 / 80, 36 and 38 us, however little there is
-// to sum.
-constexpr int kRdwMaxChunk = 512;
-int router_dw_chunk(int64_t tokens, int d_model, int n_experts) {
-  const int64_t tiles = (d_model / 128 > 0 ? d_model / 128 : 1) * ceil_div(n_experts, 64);
-  int chunk = kRdwMaxChunk;
-  while (chunk > 64 && tiles * ceil_div(tokens, chunk) < 256) chunk /= 2;
-  return chunk;
-}
+constexpr int kRdwChunk = 512;
 constexpr int kRdwStrideX = 160;  // row offset 32 banks apart: the two k rows never collide
 constexpr int kRdwStrideL = 96;
 
@@ -369,7 +359,7 @@ template <typename TX>
 __global__ __launch_bounds__(256) void router_dw_partial_kernel(const TX* __restrict__ x,
                                                                 const float* __restrict__ d_logits,
                                                                 int64_t tokens, int d_model,
-                                                                int n_experts, int chunk,
+                                                                int n_experts,
                                                                 float* __restrict__ partial) {
   __shared__ float sx[64 * kRdwStrideX];
   __shared__ float sl[64 * kRdwStrideL];
@@ -378,8 +368,8 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(const TX* __rest
   const int l32 = lane & 31, hi = lane >> 5;
   const int d0 = blockIdx.x * 128, n0 = blockIdx.y * 64;
   const int64_t c = blockIdx.z;
-  const int64_t t_begin = c * chunk;
-  const int64_t t_end = t_begin + chunk < tokens ? t_begin + chunk : tokens;
+  const int64_t t_begin = c * kRdwChunk;
+  const int64_t t_end = t_begin + kRdwChunk < tokens ? t_begin + kRdwChunk : tokens;
   f32x16 acc[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
@@ -453,8 +443,6 @@ __global__ __launch_bounds__(256) void router_dw_sum_kernel(const float* __restr
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < count;
        i += static_cast<int64_t>(gridDim.x) * 256) {
     float v = 0.0f;
-    // (in chunk order; the loads of eight chunks in flight)
-#pragma unroll 8
     for (int c = 0; c < chunks; ++c) v = v + partial[c * count + i];
     out[i] = v;
   }
@@ -570,8 +558,7 @@ extern "C" int hmoe_router_dx(const float* d_logits, const void* router_w, int w
 
 extern "C" size_t hmoe_router_dw_workspace_bytes(int64_t tokens, int d_model, int n_experts) {
   if (tokens <= 0 || d_model <= 0 || n_experts <= 0) return 0;
-  return static_cast<size_t>(hmoe::ceil_div(
-             tokens, hmoe::router_dw_chunk(tokens, d_model, n_experts))) * d_model * n_experts *
+  return static_cast<size_t>(hmoe::ceil_div(tokens, hmoe::kRdwChunk)) * d_model * n_experts *
          sizeof(float);
 }
 
@@ -588,17 +575,16 @@ extern "C" int hmoe_router_dw(const void* x, int x_dtype, const float* d_logits,
   HMOE_REQUIRE_CODE(workspace_bytes >= need, HMOE_ERR_WORKSPACE,
                     "router_dw: workspace of %zu bytes, need %zu", workspace_bytes, need);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int chunk = router_dw_chunk(tokens, d_model, n_experts);
-  const int chunks = static_cast<int>(ceil_div(tokens, chunk));
+  const int chunks = static_cast<int>(ceil_div(tokens, kRdwChunk));
   float* partial = static_cast<float*>(workspace);
   const dim3 grid(static_cast<unsigned>(d_model / 128), static_cast<unsigned>(ceil_div(n_experts, 64)),
                   static_cast<unsigned>(chunks));
   if (x_dtype == HMOE_F32)
     hipLaunchKernelGGL(router_dw_partial_kernel<float>, grid, dim3(256), 0, s,
-                       static_cast<const float*>(x), d_logits, tokens, d_model, n_experts, chunk, partial);
+                       static_cast<const float*>(x), d_logits, tokens, d_model, n_experts, partial);
   else
     hipLaunchKernelGGL(router_dw_partial_kernel<uint16_t>, grid, dim3(256), 0, s,
-                       static_cast<const uint16_t*>(x), d_logits, tokens, d_model, n_experts, chunk,
+                       static_cast<const uint16_t*>(x), d_logits, tokens, d_model, n_experts,
                        partial);
   const int64_t count = static_cast<int64_t>(d_model) * n_experts;
   hipLaunchKernelGGL(router_dw_sum_kernel, dim3(static_cast<unsigned>(std::min<int64_t>(ceil_div(count, 256), 4096))),
