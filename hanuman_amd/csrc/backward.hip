@@ -436,6 +436,92 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(const TX* __rest
   }
 }
 
+// The same partials where the tiles above are fewer than the CUs: 32 d x 32 n of
+// one chunk per workgroup, its four waves taking every fourth 32 tokens with
+// their operands straight from global memory in the MFMA's layout, a step of 16
+// MFMAs ahead (rows past the chunk read as zeros by the buffer range check),
+// added through LDS in wave order.  At 2048 tokens the 128 x 64 tiles are 8 for
+// d_model 256 / 8 experts and 96 for 1536 / 80, and took 37 and 39 us however
+// little there is to sum.
+template <typename TX>
+__global__ __launch_bounds__(256) void router_dw_split_kernel(const TX* __restrict__ x,
+                                                              const float* __restrict__ d_logits,
+                                                              int64_t tokens, int d_model,
+                                                              int n_experts,
+                                                              float* __restrict__ partial) {
+  __shared__ f32x4 part[4 * 4 * 64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hi = lane >> 5;
+  const int d0 = blockIdx.x * 32, n0 = blockIdx.y * 32;
+  const int64_t c = blockIdx.z;
+  const int64_t t_begin = c * kRdwChunk;
+  const int rows = static_cast<int>(t_begin + kRdwChunk < tokens ? kRdwChunk : tokens - t_begin);
+  const int n = n0 + l32 < n_experts ? n0 + l32 : n_experts - 1;  // past the last: never stored
+  constexpr int kXB = static_cast<int>(sizeof(TX));
+  struct Step {
+    uint32_t a[16], b[16];
+  };
+  const int a_voff = (hi * d_model + d0 + l32) * kXB;
+  const int b_voff = (hi * n_experts + n) * 4;
+  auto load = [&](Step& s, int r0) __attribute__((always_inline)) {
+    const int left = rows - r0 < 32 ? rows - r0 : 32;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<TX*>(x + (t_begin + r0) * d_model), 0, left * d_model * kXB, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(d_logits + (t_begin + r0) * n_experts), 0, left * n_experts * 4, 0x00020000);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (kXB == 4)
+        s.a[q] = __builtin_amdgcn_raw_buffer_load_b32(ra, a_voff + 2 * q * d_model * kXB, 0, 0);
+      else
+        s.a[q] = static_cast<uint32_t>(
+                     __builtin_amdgcn_raw_buffer_load_b16(ra, a_voff + 2 * q * d_model * kXB, 0, 0));
+      s.b[q] = __builtin_amdgcn_raw_buffer_load_b32(rb, b_voff + 2 * q * n_experts * 4, 0, 0);
+    }
+  };
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  auto compute = [&](const Step& s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      acc = mfma_f32_32x32x2(__uint_as_float(kXB == 4 ? s.a[q] : s.a[q] << 16), __uint_as_float(s.b[q]),
+                             acc);
+  };
+  const int n_st = (rows + 31) / 32;
+  Step s0, s1;
+  int st = wave;
+  if (st < n_st) load(s0, st * 32);
+  for (; st < n_st; st += 8) {
+    if (st + 4 < n_st) load(s1, (st + 4) * 32);
+    compute(s0);
+    if (st + 4 >= n_st) break;
+    if (st + 8 < n_st) load(s0, (st + 8) * 32);
+    compute(s1);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    f32x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = acc[4 * q + r];
+    part[(wave * 4 + q) * 64 + lane] = v;
+  }
+  __syncthreads();
+  // wave w finishes group q = w: d0 + 8 w + 4 hi + 0..3 of column n0 + l32
+  if (n0 + l32 >= n_experts) return;
+  f32x4 v = part[wave * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    const f32x4 t = part[(w * 4 + wave) * 64 + lane];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] += t[r];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    partial[(c * d_model + d0 + 8 * wave + 4 * hi + r) * n_experts + n0 + l32] = v[r];
+}
+
 __global__ __launch_bounds__(256) void router_dw_sum_kernel(const float* __restrict__ partial,
                                                             int chunks, int64_t count,
                                                             float* __restrict__ out) {
@@ -579,7 +665,18 @@ extern "C" int hmoe_router_dw(const void* x, int x_dtype, const float* d_logits,
   float* partial = static_cast<float*>(workspace);
   const dim3 grid(static_cast<unsigned>(d_model / 128), static_cast<unsigned>(ceil_div(n_experts, 64)),
                   static_cast<unsigned>(chunks));
-  if (x_dtype == HMOE_F32)
+  // fewer 128 x 64 tiles than the 256 CUs of the part
+  if (static_cast<int64_t>(grid.x) * grid.y * grid.z < 256) {
+    const dim3 split(static_cast<unsigned>(d_model / 32), static_cast<unsigned>(ceil_div(n_experts, 32)),
+                     static_cast<unsigned>(chunks));
+    if (x_dtype == HMOE_F32)
+      hipLaunchKernelGGL(router_dw_split_kernel<float>, split, dim3(256), 0, s,
+                         static_cast<const float*>(x), d_logits, tokens, d_model, n_experts, partial);
+    else
+      hipLaunchKernelGGL(router_dw_split_kernel<uint16_t>, split, dim3(256), 0, s,
+                         static_cast<const uint16_t*>(x), d_logits, tokens, d_model, n_experts,
+                         partial);
+  } else if (x_dtype == HMOE_F32)
     hipLaunchKernelGGL(router_dw_partial_kernel<float>, grid, dim3(256), 0, s,
                        static_cast<const float*>(x), d_logits, tokens, d_model, n_experts, partial);
   else
