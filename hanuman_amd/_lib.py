@@ -86,6 +86,8 @@ SIGNATURES = {
     "hmoe_swiglu_bwd": (_i32, [_vp, _vp, _vp, _i32, _i64, _i32, _vp, _vp]),
     "hmoe_pack_down_dgrad": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     "hmoe_pack_gate_up_dgrad": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp]),
+    "hmoe_pack_gate_up_train": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
+    "hmoe_pack_down_train": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
     "hmoe_grouped_dgrad_down": (_i32, [_vp, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
     "hmoe_grouped_dgrad_gate_up": (_i32, [_vp, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
     "hmoe_gather_bwd": (_i32, [_vp, _i32, _vp, _vp, _i32, _i64, _i32, _i32, _vp, _i32, _vp]),

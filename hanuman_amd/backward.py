@@ -53,6 +53,13 @@ class BackwardOperands:
         self.w_gate_up_dgrad = K.pack_gate_up_dgrad(w_gate, w_up)
         self.w_down_dgrad = K.pack_down_dgrad(w_down)
 
+    @classmethod
+    def from_packed(cls, w_gate_up_dgrad: torch.Tensor, w_down_dgrad: torch.Tensor):
+        """From operands already packed (:func:`kernels.pack_gate_up_train`)."""
+        self = cls.__new__(cls)
+        self.w_gate_up_dgrad, self.w_down_dgrad = w_gate_up_dgrad, w_down_dgrad
+        return self
+
 
 class SharedOperands:
     """Packed operands of the shared expert(s) (``moe.py:152-159``): 2-D

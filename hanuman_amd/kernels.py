@@ -825,6 +825,31 @@ def pack_gate_up_dgrad(w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor
     return out
 
 
+def pack_gate_up_train(w_gate: torch.Tensor, w_up: torch.Tensor):
+    """(:func:`pack_gate_up`, :func:`pack_gate_up_dgrad`) from one read of the masters."""
+    _check(w_gate, "w_gate", 3)
+    _check(w_up, "w_up", 3)
+    if w_gate.shape != w_up.shape or w_gate.dtype != w_up.dtype:
+        raise ValueError("w_gate and w_up must have the same shape and dtype")
+    N, D, F = w_gate.shape
+    fwd = torch.empty((N, 2 * F, D), dtype=torch.bfloat16, device=w_gate.device)
+    bwd = torch.empty((N, D, 2 * F), dtype=torch.bfloat16, device=w_gate.device)
+    call("hmoe_pack_gate_up_train", _ptr(w_gate), _ptr(w_up), _dtype_code(w_gate), N, D, F,
+         _ptr(fwd), _ptr(bwd), _stream())
+    return fwd, bwd
+
+
+def pack_down_train(w_down: torch.Tensor):
+    """(:func:`pack_down`, :func:`pack_down_dgrad`) from one read of the master."""
+    _check(w_down, "w_down", 3)
+    N, F, D = w_down.shape
+    fwd = torch.empty((N, D, F), dtype=torch.bfloat16, device=w_down.device)
+    bwd = torch.empty((N, F, D), dtype=torch.bfloat16, device=w_down.device)
+    call("hmoe_pack_down_train", _ptr(w_down), _dtype_code(w_down), N, F, D, _ptr(fwd), _ptr(bwd),
+         _stream())
+    return fwd, bwd
+
+
 def grouped_dgrad_down(d_ys: torch.Tensor, offsets: torch.Tensor, w_down_dgrad: torch.Tensor) -> torch.Tensor:
     """``dh = bf16(d_ys Wd[e]^T)`` per expert segment (VJP of ``moe.py:73``)."""
     _check(d_ys, "d_ys", 2)

@@ -103,10 +103,13 @@ class _PackCache:
                 and all(r() is t for r, t in zip(self._refs, tensors))
                 and all(self._key(t) == k for t, k in zip(tensors, self._keys)))
         if not same:
-            self._val = build()
-            self._refs = tuple(weakref.ref(t) for t in tensors)
-            self._keys = tuple(self._key(t) for t in tensors)
+            self.put(tensors, build())
         return self._val
+
+    def put(self, tensors, val):
+        self._val = val
+        self._refs = tuple(weakref.ref(t) for t in tensors)
+        self._keys = tuple(self._key(t) for t in tensors)
 
 
 def swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
@@ -212,6 +215,8 @@ class MoE:
             self.shared_w_down = Param(normal((n_shared_experts, dfs, d_model), std))
         self._routed_pack = _PackCache()
         self._shared_pack = _PackCache()
+        self._routed_bwd_pack = _PackCache()
+        self._shared_bwd_pack = _PackCache()
 
     # ---- parameters ------------------------------------------------------
     def named_params(self) -> dict:
@@ -260,12 +265,23 @@ class MoE:
         from safetensors.numpy import load_file
         self.load_state(load_file(str(path)))
 
-    def _packed_routed(self, masters=None):
+    def _packed_routed(self, masters=None, train: bool = False):
         """Packed routed-expert operands of ``masters`` (default: the current
-        parameters)."""
+        parameters).  ``train``: a backward follows, so masters that have to be
+        packed anew are read once for its operands too."""
         wg, wu, wd = masters if masters is not None else (
             self.expert_w_gate.value, self.expert_w_up.value, self.expert_w_down.value)
-        return self._routed_pack.get((wg, wu, wd), lambda: (K.pack_gate_up(wg, wu), K.pack_down(wd)))
+
+        def build():
+            if not train:
+                return K.pack_gate_up(wg, wu), K.pack_down(wd)
+            from .backward import BackwardOperands
+            gate_up, gate_up_dgrad = K.pack_gate_up_train(wg, wu)
+            down, down_dgrad = K.pack_down_train(wd)
+            self._routed_bwd_pack.put((wg, wu, wd),
+                                      BackwardOperands.from_packed(gate_up_dgrad, down_dgrad))
+            return gate_up, down
+        return self._routed_pack.get((wg, wu, wd), build)
 
     def _packed_shared(self, masters=None):
         wg, wu, wd = masters if masters is not None else (
@@ -385,7 +401,7 @@ class MoE:
                          "plan": plan, "xs": xs, "h": h, "ys": ys, "h_shared": hs, "mode": mode,
                          "rsf": rsf, "batch": B, "seq": S}
             return out.reshape(B, S, D), losses, counts, saved
-        wgu, wd = self._packed_routed()
+        wgu, wd = self._packed_routed(train=save)
         if x2.dtype == torch.bfloat16:
             # the gate/up GEMM gathers its rows from x (moe.py:56 fused)
             h = K.grouped_gate_up_gather(x2, plan, wgu)
@@ -411,16 +427,13 @@ class MoE:
         """Packed backward operands of the routed and shared experts for the
         masters ``(wg, wu, wd, swg, swu, swd)`` the forward used, cached like
         the forward's packs (rebuilt when a master changes)."""
-        if not hasattr(self, "_bwd_pack"):
-            self._bwd_pack = _PackCache()
         wg, wu, wd, swg, swu, swd = masters
         from .backward import BackwardOperands, SharedOperands
-
-        def build():
-            return (BackwardOperands(wg, wu, wd),
-                    SharedOperands(swg, swu, swd, self.n_shared_experts,
-                                   self._packed_shared((swg, swu, swd))))
-        return self._bwd_pack.get((wg, wu, wd, swg, swu, swd), build)
+        routed = self._routed_bwd_pack.get((wg, wu, wd), lambda: BackwardOperands(wg, wu, wd))
+        shared = self._shared_bwd_pack.get(
+            (swg, swu, swd), lambda: SharedOperands(swg, swu, swd, self.n_shared_experts,
+                                                    self._packed_shared((swg, swu, swd))))
+        return routed, shared
 
 
 class _MoEFunction(torch.autograd.Function):

@@ -805,6 +805,45 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoePackGateUpDgrad, PackGateUpDgradImpl,
                                   .Arg<ffi::AnyBuffer>()
                                   .Ret<ffi::Buffer<ffi::BF16>>());
 
+// Both operands from one read of the masters: wg, wu [N, D, F] -> [N, 2F, D] and
+// [N, D, 2F] bf16; wd [N, F, D] -> [N, D, F] and [N, F, D] bf16.
+static ffi::Error PackGateUpTrainImpl(hipStream_t stream, ffi::AnyBuffer wg, ffi::AnyBuffer wu,
+                                      ffi::ResultBuffer<ffi::BF16> packed,
+                                      ffi::ResultBuffer<ffi::BF16> packed_dgrad) {
+  const int d = DtypeCode(wg.element_type());
+  if (d < 0 || DtypeCode(wu.element_type()) != d) return BadDtype("hmoe_pack_gate_up_train");
+  auto dims = wg.dimensions();
+  return Status(hmoe_pack_gate_up_train(wg.untyped_data(), wu.untyped_data(), d,
+                                        static_cast<int>(dims[0]), static_cast<int>(dims[1]),
+                                        static_cast<int>(dims[2]), packed->untyped_data(),
+                                        packed_dgrad->untyped_data(), S(stream)));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoePackGateUpTrain, PackGateUpTrainImpl,
+                              ffi::Ffi::Bind()
+                                  .Ctx<ffi::PlatformStream<hipStream_t>>()
+                                  .Arg<ffi::AnyBuffer>()
+                                  .Arg<ffi::AnyBuffer>()
+                                  .Ret<ffi::Buffer<ffi::BF16>>()
+                                  .Ret<ffi::Buffer<ffi::BF16>>());
+
+static ffi::Error PackDownTrainImpl(hipStream_t stream, ffi::AnyBuffer wd,
+                                    ffi::ResultBuffer<ffi::BF16> packed,
+                                    ffi::ResultBuffer<ffi::BF16> packed_dgrad) {
+  const int d = DtypeCode(wd.element_type());
+  if (d < 0) return BadDtype("hmoe_pack_down_train");
+  auto dims = wd.dimensions();
+  return Status(hmoe_pack_down_train(wd.untyped_data(), d, static_cast<int>(dims[0]),
+                                     static_cast<int>(dims[1]), static_cast<int>(dims[2]),
+                                     packed->untyped_data(), packed_dgrad->untyped_data(),
+                                     S(stream)));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoePackDownTrain, PackDownTrainImpl,
+                              ffi::Ffi::Bind()
+                                  .Ctx<ffi::PlatformStream<hipStream_t>>()
+                                  .Arg<ffi::AnyBuffer>()
+                                  .Ret<ffi::Buffer<ffi::BF16>>()
+                                  .Ret<ffi::Buffer<ffi::BF16>>());
+
 // dh = d_ys Wd^T: d_ys [rows_cap, D] bf16, offsets, packed [N, F, D] ->
 // dh [rows_cap, F] bf16.
 static ffi::Error GroupedDgradDownImpl(hipStream_t stream, ffi::Buffer<ffi::BF16> d_ys,

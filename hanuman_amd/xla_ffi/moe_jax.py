@@ -85,6 +85,8 @@ TARGETS = {
     "hmoe_swiglu_bwd": "HmoeSwigluBwd",
     "hmoe_pack_down_dgrad": "HmoePackDownDgrad",
     "hmoe_pack_gate_up_dgrad": "HmoePackGateUpDgrad",
+    "hmoe_pack_gate_up_train": "HmoePackGateUpTrain",
+    "hmoe_pack_down_train": "HmoePackDownTrain",
     "hmoe_grouped_dgrad_down": "HmoeGroupedDgradDown",
     "hmoe_grouped_dgrad_gate_up": "HmoeGroupedDgradGateUp",
     "hmoe_gather_bwd": "HmoeGatherBwd",

@@ -443,6 +443,14 @@ int hmoe_pack_down_dgrad(const void* w_down, int w_dtype, int n_experts, int d_f
                          int d_model, void* packed, hmoe_stream_t stream);
 int hmoe_pack_gate_up_dgrad(const void* w_gate, const void* w_up, int w_dtype, int n_experts,
                             int d_model, int d_ff, void* packed, hmoe_stream_t stream);
+/* The forward's and the backward's operand from one read of the masters (a
+ * training step packs both anew): hmoe_pack_gate_up + hmoe_pack_gate_up_dgrad,
+ * hmoe_pack_down + hmoe_pack_down_dgrad, the same bits. */
+int hmoe_pack_gate_up_train(const void* w_gate, const void* w_up, int w_dtype, int n_experts,
+                            int d_model, int d_ff, void* packed, void* packed_dgrad,
+                            hmoe_stream_t stream);
+int hmoe_pack_down_train(const void* w_down, int w_dtype, int n_experts, int d_ff, int d_model,
+                         void* packed, void* packed_dgrad, hmoe_stream_t stream);
 
 /* dh = bf16(d_ys Wd[e]^T) per expert segment (the VJP of moe.py:73 with
  * respect to h): d_ys [rows_cap, D], dh [rows_cap, F] bf16, w_down_dgrad
