@@ -36,6 +36,7 @@
 //     four LDS stages (buffer_load ... lds, three steps ahead), because the
 //     32-byte fp8 fragments leave no registers for load staging.
 #include <atomic>
+#include <algorithm>
 #include <cmath>
 
 #include "hmoe_common.h"
@@ -1233,6 +1234,12 @@ __device__ __forceinline__ f32x16 few_mfma_scaled(const i32x8& b, const i32x8& a
 // waves the others only load.  Tiles are numbered and dealt to the XCDs as in
 // the 256 x 256 kernels, and every output is summed in the same K order, so
 // the results are the same bits.
+//
+// Dense groups (the shared experts) may follow the experts in one launch:
+// FewDense's `groups` of `rows` rows each, at rows base.. of C (and of A, unless
+// it is gathered: then row r of each is row r of A), with weights of the same
+// shape.  On their own their few tiles leave most CUs idle behind one tile's
+// latency.
 enum FewEpi { kFewPlain = 0, kFewSwiglu = 1, kFewDSwiglu = 2, kFewSwigluQ = 3 };
 enum FewElem { kFewBf16 = 0, kFewE4m3 = 1, kFewE4m3Mx = 2 };  // Mx: block-scaled A
 
@@ -1248,17 +1255,26 @@ struct FewCfg {
   static_assert((kStages - 2) * (kNA + kNB) < 63, "vmcnt is a 6-bit count");
 };
 
+struct FewDense {
+  const uint8_t* B;
+  int groups, rows, base;
+};
+
 template <int BM>
-__device__ __forceinline__ int scan_few_tiles(const int32_t* __restrict__ offsets, int n_experts,
-                                              int32_t* toff, int32_t* tstart, int32_t* scan_tmp) {
+__device__ __forceinline__ int scan_few_tiles(const int32_t* __restrict__ offsets, int n_routed,
+                                              int dense_groups, int dense_rows, int32_t* toff,
+                                              int32_t* tstart, int32_t* scan_tmp) {
+  const int n_experts = n_routed + dense_groups;
+  const int dense_tiles = (dense_rows + BM - 1) / BM;
   const int tid = threadIdx.x;
   const int per = (n_experts + kThreads - 1) / kThreads;
-  for (int e = tid; e <= n_experts; e += kThreads) toff[e] = offsets[e];
+  for (int e = tid; e <= n_routed; e += kThreads) toff[e] = offsets[e];
   __syncthreads();
   int sum = 0;
   for (int j = 0; j < per; ++j) {
     const int e = tid * per + j;
-    if (e < n_experts) sum += (toff[e + 1] - toff[e] + BM - 1) / BM;
+    if (e < n_routed) sum += (toff[e + 1] - toff[e] + BM - 1) / BM;
+    else if (e < n_experts) sum += dense_tiles;
   }
   scan_tmp[tid] = sum;
   __syncthreads();
@@ -1273,12 +1289,17 @@ __device__ __forceinline__ int scan_few_tiles(const int32_t* __restrict__ offset
     const int e = tid * per + j;
     if (e < n_experts) {
       tstart[e] = run;
-      run += (toff[e + 1] - toff[e] + BM - 1) / BM;
+      run += e < n_routed ? (toff[e + 1] - toff[e] + BM - 1) / BM : dense_tiles;
     }
   }
   if (tid == kThreads - 1) tstart[n_experts] = scan_tmp[kThreads - 1];
   __syncthreads();
   return tstart[n_experts];
+}
+
+// The launches that take dense groups: the bf16 layer's two forward GEMMs.
+constexpr bool few_takes_dense(int elem, int epi, bool gather) {
+  return elem == kFewBf16 && (gather ? epi == kFewSwiglu : epi == kFewPlain);
 }
 
 template <int ELEM, int EPI, bool GATHER, int BM, int BN>
@@ -1287,7 +1308,7 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
     const float* __restrict__ a_scale, const float* __restrict__ b_scale,
     const int32_t* __restrict__ offsets, int n_experts, int kdim, int ncols,
     uint16_t* __restrict__ C, int64_t ldc, const int32_t* __restrict__ gather_src, int gather_k,
-    int gather_rows, const uint16_t* __restrict__ dh, uint8_t* __restrict__ mx_exp) {
+    int gather_rows, const uint16_t* __restrict__ dh, uint8_t* __restrict__ mx_exp, FewDense dense) {
   typedef FewCfg<ELEM, BM, BN> Cfg;
   constexpr bool kFp8 = ELEM != kFewBf16;
   constexpr int kNA = Cfg::kNA, kNB = Cfg::kNB, kStages = Cfg::kStages;
@@ -1295,6 +1316,7 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
   constexpr int kWM = 4 / kWN;                             // row groups
   constexpr int kRB = BM / 32;
   constexpr int kFR = kRB >= kWM ? kRB / kWM : 1;          // row fragments per wave
+  constexpr bool kDense = few_takes_dense(ELEM, EPI, GATHER);
   static_assert(!(ELEM == kFewE4m3Mx && GATHER), "the block-scaled A operand is not gathered");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ int32_t toff[kMaxExperts + 1];
@@ -1304,8 +1326,10 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_tiles_n = ncols / BN;
+  const int n_groups = kDense ? n_experts + dense.groups : n_experts;
   const int total = __builtin_amdgcn_readfirstlane(
-      scan_few_tiles<BM>(offsets, n_experts, toff, tstart, scan_tmp) * n_tiles_n);
+      scan_few_tiles<BM>(offsets, n_experts, n_groups - n_experts, dense.rows, toff, tstart, scan_tmp) *
+      n_tiles_n);
   const int xcd = blockIdx.x % kNumXcd;
   const int per_xcd = gridDim.x / kNumXcd;
   const int slot = blockIdx.x / kNumXcd;
@@ -1320,11 +1344,12 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
   // Tile t: as decode_tile_grouped (groups of 8 row tiles, row tile fastest).
   struct Tile {
     int e, row0, row_end, n0;
+    int seg0;  // the segment's first row
   };
   auto decode = [&](int t) __attribute__((always_inline)) {
     constexpr int G = 8;
     const int m_any = t / n_tiles_n;
-    int l = 0, h = n_experts;
+    int l = 0, h = n_groups;
     while (h - l > 1) {
       const int mid = (l + h) >> 1;
       if (tstart[mid] <= m_any) l = mid; else h = mid;
@@ -1339,8 +1364,14 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
     const int n_tile = v / gm;
     Tile r;
     r.e = e;
-    r.row0 = __builtin_amdgcn_readfirstlane(toff[e]) + (g * G + (v - n_tile * gm)) * BM;
-    r.row_end = __builtin_amdgcn_readfirstlane(toff[e + 1]);
+    if (kDense && e >= n_experts) {
+      r.seg0 = dense.base + (e - n_experts) * dense.rows;
+      r.row_end = r.seg0 + dense.rows;
+    } else {
+      r.seg0 = __builtin_amdgcn_readfirstlane(toff[e]);
+      r.row_end = __builtin_amdgcn_readfirstlane(toff[e + 1]);
+    }
+    r.row0 = r.seg0 + (g * G + (v - n_tile * gm)) * BM;
     r.n0 = n_tile * BN;
     return r;
   };
@@ -1362,11 +1393,21 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_few(
   int ld_t = first, ld_kb = 0, ld_g = 0, ld_slot = 0;
   auto set_load_tile = [&](int t) __attribute__((always_inline)) {
     const Tile q = decode(t);
+    const bool is_dense = kDense && q.e >= n_experts;  // uniform
+    const uint8_t* const bw = is_dense ? dense.B : B;
     b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(B + (static_cast<int64_t>(q.e) * ncols + q.n0) * row_bytes), 0,
-        BN * row_bytes, kBufferWord3);
+        const_cast<uint8_t*>(
+            bw + (static_cast<int64_t>(is_dense ? q.e - n_experts : q.e) * ncols + q.n0) * row_bytes),
+        0, BN * row_bytes, kBufferWord3);
     const int lim = q.row_end - 1 - q.row0;  // rows past the segment repeat its last one
-    if constexpr (GATHER) {
+    if (GATHER && is_dense) {
+#pragma unroll
+      for (int j = 0; j < kNA; ++j) {
+        const int r = 8 * (wave * kNA + j) + l8;
+        a_voff[j] = gather_offset(q.row0 - q.seg0 + (r < lim ? r : lim), row_bytes,
+                                  ((lane & 7) ^ lds_swz(r)) * 16);
+      }
+    } else if constexpr (GATHER) {
       typedef const __attribute__((address_space(4))) int32_t* scalar_ptr;
       const scalar_ptr src = (scalar_ptr)(uintptr_t)gather_src;
 #pragma unroll
@@ -2466,22 +2507,37 @@ int allow_dynamic_lds(int dev) {
 //     39.6 -> 31.3 (128 x 256); 16384 rows, D 2048, F 1024 121.5 against 144.7;
 //   e4m3, 32 experts, D 4096, F 2048, top-4: 100 tokens 142.8 -> 115.3 and 56.5
 //     -> 42.7; 1600 tokens 159.9 against 172.9: old.
-void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int cus, int* bm, int* bn) {
+//
+//
+// Dense groups (in a launch of the few-rows kernel only) add their tiles and
+// their weights; the few tiles past whole rounds then matter, so there full
+// rounds share the streaming time and the last one takes a tile's own time at
+// least.  *units, if asked for, is that estimate for the shape taken.
+void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int cus, int* bm, int* bn,
+                 int dense_groups = 0, int64_t dense_rows = 0, double* units = nullptr) {
   const double n_eff = rows < n_experts ? static_cast<double>(rows) : n_experts;
   const double mean = rows / n_eff;
   const double ks = row_bytes / 128.0;
-  const double floor = n_eff * ncols * ks / (5.5e6 / 128.0) / 0.002667;
+  const double floor = (n_eff + dense_groups) * ncols * ks / (5.5e6 / 128.0) / 0.002667;
   static const int kShapes[][2] = {{256, 256}, {128, 256}, {128, 128}, {64, 256}, {64, 128},
                                    {64, 64},   {32, 256},  {32, 128},  {32, 64}};
   double best = 0.0;
   for (const auto& sh : kShapes) {
     const bool old = sh[0] == 256;
+    if (dense_groups > 0) {
+      // weights read twice for a second row tile measured slower than 128 rows
+      // (layer of 64 experts, D 2048, F 1024, 640 tokens: 287 us against 263)
+      if (old || (sh[0] < 128 && n_eff > 1.0 && mean + std::sqrt(mean) > sh[0])) continue;
+    }
     double mt;
     if (n_experts == 1)
       mt = std::ceil(mean / sh[0]);
     else
       mt = n_eff * (mean + 1.5 * std::sqrt(mean) <= sh[0] ? 1.0 : mean / sh[0] + 0.5);
-    double cost = std::ceil(mt * (ncols / sh[1]) / cus) * (ks * (sh[0] + sh[1]) + 750.0);
+    const double dense_mt = dense_groups * std::ceil(static_cast<double>(dense_rows) / sh[0]);
+    const double tile = ks * (sh[0] + sh[1]) + 750.0;
+    const double tiles = std::ceil((mt + dense_mt) * (ncols / sh[1]));
+    double cost = std::ceil(tiles / cus) * tile;
     double least = floor * (old ? 1.4 : 1.15);
     if (!old) {
       // shapes at the floor differ by little: weights read again for a second
@@ -2489,9 +2545,15 @@ void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int 
       least *= 1.0 + 0.15 * (mt / n_eff - 1.0) + 0.0004 * sh[0] +
                (sh[1] == 64 ? 0.2 : (sh[1] == 128) == (ks >= 32.0) ? 0.0 : 0.01);
     }
-    if (n_experts > 1 && cost < least) cost = least;
+    const double full = std::floor(tiles / cus), rest = tiles - full * cus;
+    const double stream = n_experts > 1 || dense_groups > 0 ? least / tiles : 0.0;
+    const double rounds = full * std::max(tile, stream * cus) +
+                          (rest > 0.0 ? std::max(tile, stream * rest) : 0.0);
+    if (dense_groups > 0) cost = rounds;
+    else if (n_experts > 1 && cost < least) cost = least;
     if (best == 0.0 || cost < best) {
       best = cost;
+      if (units != nullptr) *units = rounds;
       *bm = sh[0];
       *bn = sh[1];
     }
@@ -2504,7 +2566,7 @@ int launch_few_tile(int grid, int dev, hipStream_t s, const uint8_t* a, const ui
                     const float* a_scale, const float* b_scale, const int32_t* offsets,
                     int n_experts, int kdim, int ncols, uint16_t* c, int64_t ldc,
                     const int32_t* gather_src, int gather_k, int gather_rows, const uint16_t* dh,
-                    uint8_t* mx_exp) {
+                    uint8_t* mx_exp, FewDense dense) {
   constexpr int kLds = FewCfg<ELEM, BM, BN>::kLds;
   static std::atomic<uint64_t> done{0};  // devices whose LDS limit is set
   const uint64_t bit = dev >= 0 && dev < 64 ? uint64_t(1) << dev : 0;
@@ -2517,7 +2579,7 @@ int launch_few_tile(int grid, int dev, hipStream_t s, const uint8_t* a, const ui
   }
   hipLaunchKernelGGL((grouped_gemm_few<ELEM, EPI, GATHER, BM, BN>), dim3(grid), dim3(kThreads), kLds, s,
                      a, b, a_scale, b_scale, offsets, n_experts, kdim, ncols, c, ldc, gather_src,
-                     gather_k, gather_rows, dh, mx_exp);
+                     gather_k, gather_rows, dh, mx_exp, dense);
   return HMOE_OK;
 }
 
@@ -2561,7 +2623,8 @@ int launch_grouped(bool swiglu, bool fp8, const void* A, const void* B, const fl
   if (bm != kBM && (!fp8 || kdim % 128 == 0)) {
 #define HMOE_LAUNCH_FEW(EL, EP, GA)                                                             \
   rc = launch_few<EL, EP, GA>(bm, bn, grid, dev, s, a, b, a_scale, b_scale, offsets, n_experts, kdim, \
-                              ncols, c, ldc, gather_src, gather_k, gather_rows, dswiglu_dh, mx_exp)
+                              ncols, c, ldc, gather_src, gather_k, gather_rows, dswiglu_dh, mx_exp, \
+                              FewDense{nullptr, 0, 0, 0})
     int rc = HMOE_OK;
     const bool ga = gather_src != nullptr;
     if (fp8) {
@@ -2624,6 +2687,43 @@ int launch_grouped(bool swiglu, bool fp8, const void* A, const void* B, const fl
 #undef HMOE_LAUNCH_REGS
   }
   return check_launch(what);
+}
+
+// The experts' rows and n_dense dense groups of `tokens` rows in one launch of
+// the few-rows kernel (bf16): gate/up gathered through perm_src, or down with
+// perm_src null.
+int launch_with_dense(bool swiglu, const void* A, int64_t tokens, int top_k, const int32_t* perm_src,
+                      const int32_t* offsets, int n_experts, int64_t rows_cap, int kdim, int ncols,
+                      const void* B, const void* dense_b, int n_dense, void* C, int64_t ldc,
+                      hipStream_t s, const char* what) {
+  const int64_t rows = rows_cap + n_dense * tokens;
+  HMOE_REQUIRE(rows < (int64_t(1) << 31), "%s: rows must fit in int32", what);
+  HMOE_REQUIRE((ceil_div(rows, 32) + n_experts + n_dense) * (ncols / 64) < (int64_t(1) << 31),
+               "%s: too many tiles", what);
+  HMOE_REQUIRE(int64_t{256} * kdim * 2 < (int64_t(1) << 31), "%s: reduction dimension too large", what);
+  HMOE_REQUIRE(int64_t{256} * ldc * 2 < (int64_t(1) << 31), "%s: output rows too wide", what);
+  int dev = 0, grid = 0, bm = 0, bn = 0;
+  if (int rc = persistent_grid(s, &grid, &dev)) return rc;
+  choose_tile(rows_cap > 0 ? rows_cap : 1, n_experts, static_cast<int64_t>(kdim) * 2, ncols, grid, &bm,
+              &bn, n_dense, tokens);
+  const FewDense dense{static_cast<const uint8_t*>(dense_b), n_dense, static_cast<int>(tokens),
+                       static_cast<int>(rows_cap)};
+  const uint8_t* a = static_cast<const uint8_t*>(A);
+  const uint8_t* b = static_cast<const uint8_t*>(B);
+  uint16_t* c = static_cast<uint16_t*>(C);
+  const float* no_scale = nullptr;
+  const uint16_t* no_dh = nullptr;
+  uint8_t* no_exp = nullptr;
+  int rc;
+  if (swiglu)
+    rc = launch_few<kFewBf16, kFewSwiglu, true>(bm, bn, grid, dev, s, a, b, no_scale, no_scale, offsets,
+                                                n_experts, kdim, ncols, c, ldc, perm_src, top_k,
+                                                static_cast<int>(tokens), no_dh, no_exp, dense);
+  else
+    rc = launch_few<kFewBf16, kFewPlain, false>(bm, bn, grid, dev, s, a, b, no_scale, no_scale, offsets,
+                                                n_experts, kdim, ncols, c, ldc, perm_src, 1, 1, no_dh,
+                                                no_exp, dense);
+  return rc != HMOE_OK ? rc : check_launch(what);
 }
 
 }  // namespace
@@ -2690,6 +2790,100 @@ extern "C" int hmoe_grouped_down(const void* h, const int32_t* offsets, int n_ex
   return launch_grouped(false, false, h, w_down_packed, nullptr, nullptr, offsets, n_experts,
                         rows_cap, d_ff, d_model, ys, d_model, static_cast<hipStream_t>(stream),
                         "hmoe_grouped_down");
+}
+
+namespace hmoe {
+namespace {
+// Whether the shared experts join the routed launches.  While an expert has
+// few rows they always gain: a shared expert alone is 16..40 tiles and two
+// launches of mostly latency.  Past kJoinRows the joined launch's last round of
+// tiles can cost more than the two launches, so there the estimates decide, by
+// a margin of 3%.  Whole layer calls, us, separate -> joined, one shared expert:
+//   64 experts top-8, D 2048, F 1024: 1 token 124 -> 98, 48 239 -> 226, 333
+//     251 -> 235; 1500 (always 256 x 256 separate) 325, joined 378;
+//   80 experts top-8, D 1536, F 768: 48 tokens 178 -> 152, 333 187 -> 173, 900
+//     (90 rows) 213, joined 216; 1200 271 -> 237;
+//   16 experts top-2, D 1024, F 2048: 1..777 tokens 130 -> 100;
+// and two shared experts: 48 tokens of the first 278 -> 234, 333 of the second
+// 229 -> 218.
+constexpr double kJoinRows = 48.0;
+constexpr double kLaunchUnits = 1500.0;  // a launch more, about 4 us of the estimate's units
+}  // namespace
+}  // namespace hmoe
+
+extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t rows_cap, int d_model,
+                                         int d_ff, int n_shared, hmoe_stream_t stream) {
+  using namespace hmoe;
+  if (tokens < 1 || rows_cap < 1 || n_experts < 1 || n_shared < 1 || d_model < 1 || d_ff < 1) return 0;
+  if (static_cast<int64_t>(n_experts) + n_shared > kMaxExperts) return 0;
+  if (tokens * d_model * 2 >= (int64_t(1) << 31)) return 0;
+  if (rows_cap + n_shared * tokens >= (int64_t(1) << 31)) return 0;
+  int dev = 0, grid = 0;
+  if (persistent_grid(static_cast<hipStream_t>(stream), &grid, &dev) != HMOE_OK) return 0;
+  double separate = 0.0, joined = 0.0;
+  for (int gemm = 0; gemm < 2; ++gemm) {
+    const int64_t row_bytes = int64_t{2} * (gemm == 0 ? d_model : d_ff);
+    const int ncols = gemm == 0 ? 2 * d_ff : d_model;
+    if (ncols < 256) return 0;
+    int bm = 0, bn = 0;
+    double routed = 0.0, dense = 0.0, both = 0.0;
+    choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, 0, 0, &routed);
+    if (bm == kBM) return 0;
+    choose_tile(tokens, 1, row_bytes, ncols, grid, &bm, &bn, 0, 0, &dense);
+    choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, n_shared, tokens, &both);
+    separate += routed + n_shared * (dense + kLaunchUnits);
+    joined += both;
+  }
+  if (rows_cap <= kJoinRows * n_experts) return 1;
+  return joined * 1.03 < separate ? 1 : 0;
+}
+
+extern "C" int hmoe_grouped_gate_up_gather_shared(
+    const void* x, int64_t tokens, int top_k, const int32_t* perm_src, const int32_t* offsets,
+    int n_experts, int64_t rows_cap, int d_model, int d_ff, const void* w_gate_up_packed,
+    const void* shared_gate_up_packed, int n_shared, void* h, hmoe_stream_t stream) {
+  using namespace hmoe;
+  HMOE_REQUIRE(n_experts >= 1 && n_shared >= 1 && n_experts <= kMaxExperts - n_shared,
+               "grouped_gate_up_gather_shared: need n_experts >= 1, n_shared >= 1 and at most %d together "
+               "(got %d, %d)", kMaxExperts, n_experts, n_shared);
+  HMOE_REQUIRE(rows_cap >= 0 && tokens >= 0 && top_k >= 1 && (tokens >= 1 || rows_cap == 0),
+               "grouped_gate_up_gather_shared: need rows_cap >= 0, tokens >= 0, top_k >= 1 (tokens >= 1 "
+               "with rows)");
+  HMOE_REQUIRE_CODE(d_model % kBK == 0 && d_model >= kBK, HMOE_ERR_UNSUPPORTED,
+                    "grouped_gate_up_gather_shared: d_model must be a multiple of %d (got %d)", kBK,
+                    d_model);
+  HMOE_REQUIRE_CODE((2 * d_ff) % kBN == 0 && d_ff > 0, HMOE_ERR_UNSUPPORTED,
+                    "grouped_gate_up_gather_shared: d_ff must be a multiple of %d (got %d)", kBN / 2,
+                    d_ff);
+  HMOE_REQUIRE(tokens * d_model * 2 < (int64_t(1) << 31),
+               "grouped_gate_up_gather_shared: x must be smaller than 2 GiB");
+  if (rows_cap == 0 && tokens == 0) return HMOE_OK;
+  HMOE_REQUIRE(x && perm_src && offsets && w_gate_up_packed && shared_gate_up_packed && h,
+               "grouped_gate_up_gather_shared: null pointer argument");
+  return launch_with_dense(true, x, tokens, top_k, perm_src, offsets, n_experts, rows_cap, d_model,
+                           2 * d_ff, w_gate_up_packed, shared_gate_up_packed, n_shared, h, d_ff,
+                           static_cast<hipStream_t>(stream), "hmoe_grouped_gate_up_gather_shared");
+}
+
+extern "C" int hmoe_grouped_down_shared(const void* h, const int32_t* offsets, int n_experts,
+                                        int64_t rows_cap, int64_t tokens, int d_ff, int d_model,
+                                        const void* w_down_packed, const void* shared_down_packed,
+                                        int n_shared, void* ys, hmoe_stream_t stream) {
+  using namespace hmoe;
+  HMOE_REQUIRE(n_experts >= 1 && n_shared >= 1 && n_experts <= kMaxExperts - n_shared,
+               "grouped_down_shared: need n_experts >= 1, n_shared >= 1 and at most %d together "
+               "(got %d, %d)", kMaxExperts, n_experts, n_shared);
+  HMOE_REQUIRE(rows_cap >= 0 && tokens >= 0, "grouped_down_shared: rows_cap and tokens must be >= 0");
+  HMOE_REQUIRE_CODE(d_ff % kBK == 0 && d_ff >= kBK, HMOE_ERR_UNSUPPORTED,
+                    "grouped_down_shared: d_ff must be a multiple of %d (got %d)", kBK, d_ff);
+  HMOE_REQUIRE_CODE(d_model % kBN == 0 && d_model > 0, HMOE_ERR_UNSUPPORTED,
+                    "grouped_down_shared: d_model must be a multiple of %d (got %d)", kBN, d_model);
+  if (rows_cap == 0 && tokens == 0) return HMOE_OK;
+  HMOE_REQUIRE(h && offsets && w_down_packed && shared_down_packed && ys,
+               "grouped_down_shared: null pointer argument");
+  return launch_with_dense(false, h, tokens, 1, nullptr, offsets, n_experts, rows_cap, d_ff, d_model,
+                           w_down_packed, shared_down_packed, n_shared, ys, d_model,
+                           static_cast<hipStream_t>(stream), "hmoe_grouped_down_shared");
 }
 
 namespace hmoe {

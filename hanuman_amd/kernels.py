@@ -330,6 +330,48 @@ def grouped_down(h: torch.Tensor, offsets: torch.Tensor, w_down: torch.Tensor,
     return ys
 
 
+def shared_joins(plan: Plan, tokens: int, w_gate_up: torch.Tensor, shared_gate_up: torch.Tensor) -> bool:
+    """Whether the shared experts belong into the routed experts' GEMM launches
+    (:func:`grouped_swiglu_shared`): equal weight shapes and few rows an expert."""
+    N, F2, D = w_gate_up.shape
+    if tuple(shared_gate_up.shape[1:]) != (F2, D):
+        return False
+    return _lib.lib().hmoe_grouped_shared_joins(tokens, N, plan.rows_cap, D, F2 // 2,
+                                                shared_gate_up.shape[0], _stream()) == 1
+
+
+def grouped_swiglu_shared(x: torch.Tensor, plan: Plan, w_gate_up: torch.Tensor,
+                          w_down: torch.Tensor, shared_gate_up: torch.Tensor,
+                          shared_down: torch.Tensor):
+    """``(ys, shared)``: :func:`grouped_gate_up_gather` and :func:`grouped_down` with
+    the shared experts (``moe.py:152-168``; packed ``[n, 2F, D]`` and ``[n, D, F]``)
+    as further groups of the same two launches; ``ys [rows_cap, D]`` and ``shared
+    [n, T, D]`` are parts of one buffer."""
+    _check(x, "x", 2)
+    for t, n in ((w_gate_up, "w_gate_up"), (w_down, "w_down"), (shared_gate_up, "shared_gate_up"),
+                 (shared_down, "shared_down")):
+        _check(t, n, 3)
+        if t.dtype != torch.bfloat16:
+            raise TypeError("grouped_swiglu_shared takes bf16 operands")
+    T, D = x.shape
+    N, F2, D2 = w_gate_up.shape
+    n = shared_gate_up.shape[0]
+    if (x.dtype != torch.bfloat16 or D2 != D or plan.n_experts != N
+            or plan.slot_pos.numel() != T * plan.top_k or tuple(w_down.shape) != (N, D, F2 // 2)
+            or tuple(shared_gate_up.shape) != (n, F2, D)
+            or tuple(shared_down.shape) != (n, D, F2 // 2)):
+        raise ValueError("grouped_swiglu_shared: inconsistent shapes or dtypes")
+    R = plan.rows_cap
+    h = torch.empty((R + n * T, F2 // 2), dtype=torch.bfloat16, device=x.device)
+    ys = torch.empty((R + n * T, D), dtype=torch.bfloat16, device=x.device)
+    call("hmoe_grouped_gate_up_gather_shared", _ptr(x), T, plan.top_k, _ptr(plan.perm_src),
+         _ptr(plan.offsets), N, R, D, F2 // 2, _ptr(w_gate_up), _ptr(shared_gate_up), n, _ptr(h),
+         _stream())
+    call("hmoe_grouped_down_shared", _ptr(h), _ptr(plan.offsets), N, R, T, F2 // 2, D, _ptr(w_down),
+         _ptr(shared_down), n, _ptr(ys), _stream())
+    return ys[:R], ys[R:].view(n, T, D)
+
+
 FUSED_STATUS_WORD = 8   # uint32 word of the fused launch's workspace: bit 0 = a wait gave up
 
 

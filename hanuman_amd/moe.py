@@ -284,15 +284,19 @@ class MoE:
         return self._routed_pack.get((wg, wu, wd), build)
 
     def _packed_shared(self, masters=None):
+        """One ``(gate_up, down)`` of packed operands per shared expert."""
+        gate_up, down = self._packed_shared_stack(masters)
+        return [(gate_up[i:i + 1], down[i:i + 1]) for i in range(self.n_shared_experts)]
+
+    def _packed_shared_stack(self, masters=None):
+        """The shared experts' packed operands, one stack each."""
         wg, wu, wd = masters if masters is not None else (
             self.shared_w_gate.value, self.shared_w_up.value, self.shared_w_down.value)
 
         def build():
-            if self.n_shared_experts == 1:
-                return [(K.pack_gate_up(wg.unsqueeze(0).contiguous(), wu.unsqueeze(0).contiguous()),
-                         K.pack_down(wd.unsqueeze(0).contiguous()))]
-            return [(K.pack_gate_up(wg[i:i + 1].contiguous(), wu[i:i + 1].contiguous()),
-                     K.pack_down(wd[i:i + 1].contiguous())) for i in range(self.n_shared_experts)]
+            stack = [(w.unsqueeze(0) if self.n_shared_experts == 1 else w).contiguous()
+                     for w in (wg, wu, wd)]
+            return K.pack_gate_up(stack[0], stack[1]), K.pack_down(stack[2])
         return self._shared_pack.get((wg, wu, wd), build)
 
     # ---- forward -----------------------------------------------------------
@@ -318,6 +322,10 @@ class MoE:
             if hs is not None:
                 hs.append(h)
             outs.append(K.grouped_down(h, off, wd))
+        return self._shared_mean(outs)
+
+    def _shared_mean(self, outs) -> torch.Tensor:
+        """The bf16 output of one shared expert, or the float32 mean over several."""
         if len(outs) == 1:
             return outs[0]
         acc = torch.zeros_like(outs[0], dtype=torch.float32)
@@ -402,6 +410,14 @@ class MoE:
                          "rsf": rsf, "batch": B, "seq": S}
             return out.reshape(B, S, D), losses, counts, saved
         wgu, wd = self._packed_routed(train=save)
+        if x2.dtype == torch.bfloat16 and not save and self.n_shared_experts > 0:
+            # few rows an expert: the shared experts' tiles in the routed launches
+            sgu, sdown = self._packed_shared_stack()
+            if K.shared_joins(plan, T, wgu, sgu):
+                ys, outs = K.grouped_swiglu_shared(x2, plan, wgu, wd, sgu, sdown)
+                out = K.combine(ys, plan, gates, self._shared_mean(outs), torch.float32)
+                losses, counts = K.router_aux(logits, top_idx, B, S)
+                return out.reshape(B, S, D), losses, counts, None
         if x2.dtype == torch.bfloat16:
             # the gate/up GEMM gathers its rows from x (moe.py:56 fused)
             h = K.grouped_gate_up_gather(x2, plan, wgu)

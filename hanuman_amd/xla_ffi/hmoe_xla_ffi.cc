@@ -364,6 +364,58 @@ XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoeGroupedDown, GroupedDownImpl,
                                   .Arg<ffi::Buffer<ffi::U8>>()
                                   .Ret<ffi::Buffer<ffi::BF16>>());
 
+// The shared experts in the routed experts' launches: x [T, D], perm_src, offsets, packed gate/up
+// of the experts and of the n_shared shared ones, h [rows_cap + n_shared T, F].
+static ffi::Error GroupedGateUpGatherSharedImpl(
+    hipStream_t stream, ffi::Buffer<ffi::BF16> x, ffi::Buffer<ffi::S32> perm_src,
+    ffi::Buffer<ffi::S32> offsets, ffi::Buffer<ffi::U8> w, ffi::Buffer<ffi::U8> w_shared,
+    int64_t top_k, int64_t n_shared, ffi::ResultBuffer<ffi::BF16> h) {
+  const int64_t rows_cap = static_cast<int64_t>(perm_src.element_count());
+  const int n = static_cast<int>(offsets.element_count() - 1);
+  if (Rows(*h) != rows_cap + n_shared * Rows(x))
+    return ffi::Error(ffi::ErrorCode::kInvalidArgument,
+                      "h must have rows_cap + n_shared * tokens rows");
+  return Status(hmoe_grouped_gate_up_gather_shared(
+      x.untyped_data(), Rows(x), static_cast<int>(top_k), perm_src.typed_data(),
+      offsets.typed_data(), n, rows_cap, static_cast<int>(Cols(x)), static_cast<int>(Cols(*h)),
+      w.untyped_data(), w_shared.untyped_data(), static_cast<int>(n_shared), h->untyped_data(),
+      S(stream)));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoeGroupedGateUpGatherShared, GroupedGateUpGatherSharedImpl,
+                              ffi::Ffi::Bind()
+                                  .Ctx<ffi::PlatformStream<hipStream_t>>()
+                                  .Arg<ffi::Buffer<ffi::BF16>>()
+                                  .Arg<ffi::Buffer<ffi::S32>>()
+                                  .Arg<ffi::Buffer<ffi::S32>>()
+                                  .Arg<ffi::Buffer<ffi::U8>>()
+                                  .Arg<ffi::Buffer<ffi::U8>>()
+                                  .Attr<int64_t>("top_k")
+                                  .Attr<int64_t>("n_shared")
+                                  .Ret<ffi::Buffer<ffi::BF16>>());
+
+// h of the above, offsets, packed down of the experts and of the shared ones ->
+// ys [rows_cap + n_shared T, D].
+static ffi::Error GroupedDownSharedImpl(hipStream_t stream, ffi::Buffer<ffi::BF16> h,
+                                        ffi::Buffer<ffi::S32> offsets, ffi::Buffer<ffi::U8> w,
+                                        ffi::Buffer<ffi::U8> w_shared, int64_t tokens,
+                                        int64_t n_shared, ffi::ResultBuffer<ffi::BF16> ys) {
+  return Status(hmoe_grouped_down_shared(
+      h.untyped_data(), offsets.typed_data(), static_cast<int>(offsets.element_count() - 1),
+      Rows(h) - n_shared * tokens, tokens, static_cast<int>(Cols(h)), static_cast<int>(Cols(*ys)),
+      w.untyped_data(), w_shared.untyped_data(), static_cast<int>(n_shared), ys->untyped_data(),
+      S(stream)));
+}
+XLA_FFI_DEFINE_HANDLER_SYMBOL(HmoeGroupedDownShared, GroupedDownSharedImpl,
+                              ffi::Ffi::Bind()
+                                  .Ctx<ffi::PlatformStream<hipStream_t>>()
+                                  .Arg<ffi::Buffer<ffi::BF16>>()
+                                  .Arg<ffi::Buffer<ffi::S32>>()
+                                  .Arg<ffi::Buffer<ffi::U8>>()
+                                  .Arg<ffi::Buffer<ffi::U8>>()
+                                  .Attr<int64_t>("tokens")
+                                  .Attr<int64_t>("n_shared")
+                                  .Ret<ffi::Buffer<ffi::BF16>>());
+
 // e4m3 expert GEMMs (the fp8 workload rule).
 static ffi::Error GroupedGateUpFp8Impl(hipStream_t stream, ffi::Buffer<ffi::U8> xs_q,
                                        ffi::Buffer<ffi::F32> xs_scale,

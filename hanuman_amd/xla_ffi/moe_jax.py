@@ -65,6 +65,8 @@ TARGETS = {
     "hmoe_grouped_gate_up": "HmoeGroupedGateUp",
     "hmoe_grouped_gate_up_gather": "HmoeGroupedGateUpGather",
     "hmoe_grouped_down": "HmoeGroupedDown",
+    "hmoe_grouped_gate_up_gather_shared": "HmoeGroupedGateUpGatherShared",
+    "hmoe_grouped_down_shared": "HmoeGroupedDownShared",
     "hmoe_grouped_swiglu_fused": "HmoeGroupedSwigluFused",
     "hmoe_grouped_gate_up_fp8": "HmoeGroupedGateUpFp8",
     "hmoe_grouped_gate_up_fp8_gather": "HmoeGroupedGateUpFp8Gather",

@@ -217,6 +217,27 @@ int hmoe_grouped_down(const void* h, const int32_t* offsets, int n_experts,
                       int64_t rows_cap, int d_ff, int d_model,
                       const void* w_down_packed, void* ys, hmoe_stream_t stream);
 
+/* The two GEMMs of hmoe_grouped_gate_up_gather and hmoe_grouped_down with the
+ * shared experts' (moe.py:152-168; n_shared of the same d_ff, packed one after
+ * another as one stack) in the same launches: shared expert i's rows follow
+ * the experts', at rows rows_cap + i * tokens of h and ys (both of rows_cap +
+ * n_shared * tokens rows).  The same bits as separate calls.  Worth it while
+ * the experts have few rows: hmoe_grouped_shared_joins says 1 for such sizes,
+ * 0 for others and where the entries would refuse.  n_experts + n_shared <=
+ * 1024. */
+int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t rows_cap, int d_model,
+                              int d_ff, int n_shared, hmoe_stream_t stream);
+int hmoe_grouped_gate_up_gather_shared(const void* x, int64_t tokens, int top_k,
+                                       const int32_t* perm_src, const int32_t* offsets,
+                                       int n_experts, int64_t rows_cap, int d_model, int d_ff,
+                                       const void* w_gate_up_packed,
+                                       const void* shared_gate_up_packed, int n_shared, void* h,
+                                       hmoe_stream_t stream);
+int hmoe_grouped_down_shared(const void* h, const int32_t* offsets, int n_experts,
+                             int64_t rows_cap, int64_t tokens, int d_ff, int d_model,
+                             const void* w_down_packed, const void* shared_down_packed,
+                             int n_shared, void* ys, hmoe_stream_t stream);
+
 /* The layer's whole expert FFN in one persistent launch (moe.py:56,70-74:
  * the gathered gate/up GEMM with the SwiGLU, then the down GEMM): h and ys
  * are bit-identical to hmoe_grouped_gate_up_gather followed by

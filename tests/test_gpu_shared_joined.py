@@ -1,0 +1,60 @@
+"""The shared experts' tiles in the routed experts' GEMM launches, bit for bit
+against separate launches (needs an MI355X)."""
+import pytest
+import torch
+
+from hanuman_amd import MoE
+from hanuman_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # T, K, N, d_model, d_ff, shared experts, capacity factor
+    (1, 1, 1, 256, 256, 1, None),        # one row, one expert
+    (1, 8, 64, 2048, 1024, 1, None),     # most experts empty
+    (33, 2, 16, 256, 384, 3, None),      # one row past a fragment, three shared experts
+    (48, 8, 64, 2048, 1024, 2, 1.0),     # rows dropped: the experts' rows end before the shared ones
+    (333, 8, 80, 1536, 768, 1, None),    # several row tiles of the shared expert, the last partial
+    (300, 3, 7, 512, 128, 2, 0.5),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "T%d_K%d_N%d_D%d_F%d_S%d_%s" % c)
+def test_joined_equal_separate(gpu, case):
+    T, Kk, N, D, F, n, cf = case
+    print(f"shared joined {case}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(T + N)
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16).to(gpu)
+    score = torch.rand(T, N, generator=g) + 2.0 * torch.rand(N, generator=g)
+    top = score.topk(Kk, dim=1).indices.to(torch.int32).contiguous().to(gpu)
+    plan = K.dispatch_plan(top, N, K.capacity(T, Kk, N, cf))
+    std = D ** -0.5
+
+    def weights(count):
+        wg, wu = (torch.randn(count, D, F, generator=g).to(gpu) * std for _ in range(2))
+        wd = torch.randn(count, F, D, generator=g).to(gpu) * std
+        return K.pack_gate_up(wg, wu), K.pack_down(wd)
+    wgu, wd = weights(N)
+    sgu, sdown = weights(n)
+    kept = int(plan.offsets[-1])
+    ys, shared = K.grouped_swiglu_shared(x, plan, wgu, wd, sgu, sdown)
+    torch.cuda.synchronize()
+    ref = K.grouped_down(K.grouped_gate_up_gather(x, plan, wgu), plan.offsets, wd)
+    assert torch.equal(ys[:kept], ref[:kept])
+    off = K.one_group_offsets(T, x.device)
+    for i in range(n):
+        want = K.grouped_down(K.grouped_gate_up(x, off, sgu[i:i + 1]), off, sdown[i:i + 1])
+        assert torch.equal(shared[i], want)
+
+
+@pytest.mark.parametrize("shared,d_ff_shared", [(1, None), (2, None), (1, 512)])
+def test_module_same_result(gpu, monkeypatch, shared, d_ff_shared):
+    """The module with the joined launches, and where they do not apply (another
+    d_ff of the shared expert), against its separate launches."""
+    layer = MoE(512, 256, 16, 4, shared, 0.02, 2.5, torch.bfloat16, 3, d_ff_shared=d_ff_shared)
+    x = torch.randn(2, 19, 512, device=gpu, generator=torch.Generator(gpu).manual_seed(1))
+    x = x.to(torch.bfloat16)
+    with torch.no_grad():
+        joined = layer(x)[0]
+        monkeypatch.setattr(K, "shared_joins", lambda *a: False)
+        assert torch.equal(joined, layer(x)[0])

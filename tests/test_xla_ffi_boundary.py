@@ -23,8 +23,9 @@ NO_HANDLER = {
     # XLA hands every call its buffers; the library-held scratch array is for
     # callers that cannot allocate.
     "hmoe_dispatch_plan_noalloc",
-    # a host-side query, no device work
+    # host-side queries, no device work
     "hmoe_abi_version",
+    "hmoe_grouped_shared_joins",
 }
 
 
