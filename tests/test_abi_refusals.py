@@ -243,3 +243,29 @@ def test_zero_fill_checks(lib):
     expect(lib, INVALID, "multiple of 4", "hmoe_zero_fill", P, 6, S)
     expect(lib, OK, None, "hmoe_zero_fill", None, 0, S)
     expect(lib, INVALID, "null", "hmoe_zero_fill", None, 8, S)
+
+
+def test_joined_launch_checks(lib):
+    def gate_up(n=4, r=10, d=256, f=128, t=64, shared=1, p=P):
+        return ("hmoe_grouped_gate_up_gather_shared", p, t, 2, p, p, n, r, d, f, p, p, shared, p, S)
+
+    def down(n=4, r=10, d=256, f=256, t=64, shared=1, p=P):
+        return ("hmoe_grouped_down_shared", p, p, n, r, t, f, d, p, p, shared, p, S)
+
+    for build, bad_d in ((gate_up, 100), (down, 300)):
+        expect(lib, INVALID, "n_experts", *build(n=0))
+        expect(lib, INVALID, "n_shared", *build(shared=0))
+        expect(lib, INVALID, "1024", *build(n=1024, shared=1))
+        expect(lib, UNSUPPORTED, "d_model", *build(d=bad_d))
+        expect(lib, UNSUPPORTED, "d_ff", *build(f=100))
+        expect(lib, INVALID, "rows_cap", *build(r=-1))
+        expect(lib, OK, None, *build(r=0, t=0, p=None))
+        expect(lib, INVALID, "null", *build(p=None))
+        expect(lib, INVALID, "int32", *build(r=1 << 31))
+    expect(lib, INVALID, "2 GiB", *gate_up(t=1 << 20, d=1024))
+    # sizes that the launches above refuse, or that have no rows, do not join
+    joins = lib.hmoe_grouped_shared_joins
+    assert joins(0, 4, 0, 256, 128, 1, S) == 0
+    assert joins(1 << 20, 4, 10, 1024, 128, 1, S) == 0
+    assert joins(64, 1024, 10, 256, 128, 1, S) == 0
+    assert joins(64, 4, 10, 256, 128, 0, S) == 0
