@@ -368,10 +368,9 @@ __device__ __forceinline__ void router_select8(const float* lg, int n_tok, int w
 //     float64 ([d][token], so that a wave's operand is 64 consecutive
 //     doubles), instead of by every wave for every expert tile;
 //   * W goes from global memory straight into the registers of the one wave
-//     that owns its columns, a chunk ahead; rows past d_model come back as
-//     zeros from the buffer range check.  (Through LDS, by DMA, its reads and
-//     those of x together are more than the LDS delivers: 29 against 17 us at
-//     one token, 64 experts, d_model 2048);
+//     that owns its columns, a chunk ahead, zeros past d_model.  (Through LDS,
+//     by DMA, its reads and those of x together are more than the LDS delivers:
+//     29 against 16 us at one token, 64 experts, d_model 2048);
 //   * a wave widens the W values of a group of MFMAs before the group: between
 //     two MFMAs of the chain a conversion costs 21 cycles (it waits for the
 //     first and the second waits for it).
@@ -424,13 +423,13 @@ __device__ __forceinline__ double widen_w(uint32_t bits) {
 // row of x per wave.  They start once the router's workgroups are placed and
 // run beside them, whose float64 MFMA chains leave the memory system and most
 // of the VALU issue idle.
-template <int MT, int TOK, typename XT, typename WT, bool QX>
+template <int MT, int TOK, bool TAIL, typename XT, typename WT, bool QX>
 __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 4 : 2) void router_kernel(
     const XT* __restrict__ x, const WT* __restrict__ w, const float* __restrict__ bias,
     int64_t tokens, int d_model, int n_experts, int top_k, int mode, float rsf,
     float* __restrict__ logits, int32_t* __restrict__ top_idx, float* __restrict__ gates,
     uint8_t* __restrict__ x_q, float* __restrict__ x_scale, int router_blocks) {
-  static_assert(TOK == 16 || TOK == 4, "a chain holds 16 or 4 tokens");
+  static_assert(TOK == 16 || (TOK == 4 && !TAIL), "a chain holds 16 or 4 tokens");
   static_assert(!QX || sizeof(XT) == 2, "x is quantised from bf16");
   const int n_waves = static_cast<int>(blockDim.x) >> 6;
   if constexpr (QX) {
@@ -500,7 +499,13 @@ __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 
   };
   // W: lane (k, j) reads row 4 s + k, column n of its tile; columns past
   // n_experts repeat the last one (never stored).  The resource of a chunk
-  // starts at its first row and ends with the matrix.
+  // starts at its first row and ends with the matrix; rows past d_model are
+  // zeros from the range check, which is relied on for the vector offset only.
+  // Short chains have the step's row there (48 tokens, 64 experts, d_model 2048:
+  // 16.7 us, 18.2 with it in the scalar offset).  In long ones that spills
+  // registers (4096 tokens: 67 against 33 us), so theirs is the scalar offset:
+  // all chunks are full, or (TAIL: d_model is no multiple of the chunk, 35 us) a
+  // step past the end has an empty resource.
   const int kl = lane >> 4;
   const int tile = kGW == 1 ? wave : wave / kGW;
   const int tw = kGW == 1 ? 0 : (wave % kGW) * TOK;  // the wave's first token
@@ -509,18 +514,29 @@ __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 
   constexpr int kWB = static_cast<int>(sizeof(WT));
   const int w_voff = (kl * n_experts + n) * kWB;
   const int w_step = 4 * n_experts * kWB;
-  auto w_rsrc = [&](int c) __attribute__((always_inline)) {
-    const int64_t left = c < nchunks ? (static_cast<int64_t>(d_model) - c * kRDc) * n_experts * kWB : 0;
-    const int64_t base = c < nchunks ? static_cast<int64_t>(c) * kRDc * n_experts : 0;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<WT*>(w + base), 0,
-                                             static_cast<int>(left < 0x7fffffff ? left : 0x7fffffff),
-                                             0x00020000);
+  struct WChunk {
+    const WT* first;
+    int bytes, steps, step;  // left of the matrix; bytes from step to step
+  };
+  auto w_chunk = [&](int c) __attribute__((always_inline)) {
+    const bool any = c < nchunks;
+    const int64_t left = any ? (static_cast<int64_t>(d_model) - c * kRDc) * n_experts * kWB : 0;
+    return WChunk{w + (any ? static_cast<int64_t>(c) * kRDc * n_experts : 0),
+                  static_cast<int>(left < 0x7fffffff ? left : 0x7fffffff),
+                  any ? (d_model - c * kRDc) / 4 : 0, any || TOK == 4 ? w_step : 0};
+  };
+  auto load_w = [&](const WChunk& k, int s) __attribute__((always_inline)) {
+    const bool in = !TAIL || s < k.steps;
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<WT*>(k.first), 0, in ? k.bytes : 0, 0x00020000);
+    return TOK == 4 ? load_w_bits<WT>(r, w_voff + s * k.step, 0)
+                    : load_w_bits<WT>(r, w_voff, in ? s * k.step : 0);
   };
   uint32_t wr0[kRSteps], wr1[kRSteps];
   {
-    const __amdgpu_buffer_rsrc_t r0 = w_rsrc(0);
+    const WChunk k0 = w_chunk(0);
 #pragma unroll
-    for (int s = 0; s < kRSteps; ++s) wr0[s] = load_w_bits<WT>(r0, w_voff, s * w_step);
+    for (int s = 0; s < kRSteps; ++s) wr0[s] = load_w(k0, s);
   }
   // the lane's selection biases, long before they are needed
   constexpr int kE8 = kNP / 8, kEPL = (kNP + 63) / 64;
@@ -555,7 +571,7 @@ __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 
   auto chunk = [&](const uint32_t (&wc)[kRSteps], uint32_t (&wn)[kRSteps], int c)
       __attribute__((always_inline)) {
     const double* xc = xs + (c & 1) * (kRDc * kTB);
-    const __amdgpu_buffer_rsrc_t rn = w_rsrc(c + 1);
+    const WChunk kn = w_chunk(c + 1);
     double ac[kRGroup], an[kRGroup], bc[kRGroup], bn[kRGroup];
     auto operands = [&](int s0, double (&a)[kRGroup], double (&b)[kRGroup])
         __attribute__((always_inline)) {
@@ -568,7 +584,7 @@ __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 
 #pragma unroll
     for (int s0 = 0; s0 < kRSteps; s0 += kRGroup) {
 #pragma unroll
-      for (int q = 0; q < kRGroup; ++q) wn[s0 + q] = load_w_bits<WT>(rn, w_voff, (s0 + q) * w_step);
+      for (int q = 0; q < kRGroup; ++q) wn[s0 + q] = load_w(kn, s0 + q);
       if (s0 + kRGroup < kRSteps) operands(s0 + kRGroup, an, bn);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -908,7 +924,7 @@ struct XQuant {
   float* scale = nullptr;
 };
 
-template <int MT, int TOK, typename XT, typename WT>
+template <int MT, int TOK, bool TAIL, typename XT, typename WT>
 void launch_router_tok(const void* x, const void* w, const float* bias, int64_t tokens,
                        int d_model, int n_experts, int top_k, int mode, float rsf, float* logits,
                        int32_t* top_idx, float* gates, hipStream_t stream, XQuant xq) {
@@ -916,7 +932,7 @@ void launch_router_tok(const void* x, const void* w, const float* bias, int64_t 
   const int rblocks = static_cast<int>(ceil_div(tokens, TOK * router_groups(MT)));
   if constexpr (sizeof(XT) == 2) {
     if (xq.q != nullptr) {
-      hipLaunchKernelGGL((router_kernel<MT, TOK, XT, WT, true>),
+      hipLaunchKernelGGL((router_kernel<MT, TOK, TAIL, XT, WT, true>),
                          dim3(static_cast<unsigned>(rblocks + ceil_div(tokens, waves))),
                          dim3(64 * waves), 0, stream, static_cast<const XT*>(x),
                          static_cast<const WT*>(w), bias, tokens, d_model, n_experts, top_k, mode,
@@ -924,7 +940,7 @@ void launch_router_tok(const void* x, const void* w, const float* bias, int64_t 
       return;
     }
   }
-  hipLaunchKernelGGL((router_kernel<MT, TOK, XT, WT, false>), dim3(static_cast<unsigned>(rblocks)),
+  hipLaunchKernelGGL((router_kernel<MT, TOK, TAIL, XT, WT, false>), dim3(static_cast<unsigned>(rblocks)),
                      dim3(64 * waves), 0, stream, static_cast<const XT*>(x),
                      static_cast<const WT*>(w), bias, tokens, d_model, n_experts, top_k, mode, rsf,
                      logits, top_idx, gates, nullptr, nullptr, rblocks);
@@ -955,8 +971,8 @@ void launch_router_staged(const void* x, const void* w, const float* bias, int64
 // Chains of 4 tokens while they leave at most 1.5 waves per SIMD: they are
 // three times as fast a chain as those of 16 (d_model / 4 MFMAs of 22 instead
 // of 64 cycles) but do half the work per cycle of the float64 pipe.  Measured
-// at d_model 2048, 64 experts: 1000 tokens 18.9 against 30.3 us, 2048 26.8 /
-// 30.4, 4096 48 / 32; 32 experts (d_model 4096), 2000 tokens: 29 / 59.  A box
+// at d_model 2048, 64 experts: 1000 tokens 17.5 against 30.3 us, 2048 26.8 /
+// 30.4, 4096 48 / 32; 32 experts (d_model 4096), 2000 tokens: 27 / 59.  A device
 // whose CU count cannot be read takes 16.
 template <int MT, typename XT, typename WT>
 void launch_router(const void* x, const void* w, const float* bias, int64_t tokens, int d_model,
@@ -964,8 +980,8 @@ void launch_router(const void* x, const void* w, const float* bias, int64_t toke
                    float* gates, hipStream_t stream, XQuant xq) {
   const int waves = (n_experts + 15) / 16 * router_groups(MT);
   if (ceil_div(tokens, 4 * router_groups(MT)) * waves <= int64_t(6) * stream_cus(stream)) {
-    launch_router_tok<MT, 4, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
-                                     logits, top_idx, gates, stream, xq);
+    launch_router_tok<MT, 4, false, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
+                                            logits, top_idx, gates, stream, xq);
     return;
   }
   if constexpr (MT == 2) {
@@ -975,8 +991,12 @@ void launch_router(const void* x, const void* w, const float* bias, int64_t toke
       return;
     }
   }
-  launch_router_tok<MT, 16, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
-                                    logits, top_idx, gates, stream, xq);
+  if (d_model % (4 * router_steps(MT, 16)) == 0)
+    launch_router_tok<MT, 16, false, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
+                                             logits, top_idx, gates, stream, xq);
+  else
+    launch_router_tok<MT, 16, true, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
+                                            logits, top_idx, gates, stream, xq);
 }
 
 template <int MT>

@@ -56,3 +56,25 @@ def test_router_chains_bit_exact(gpu, case):
     for name, got, ref in (("logits", logits, logits_ref), ("gates", g, g_ref)):
         assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32)), name
     assert np.array_equal(idx.cpu().numpy(), idx_ref)
+
+
+@pytest.mark.parametrize("D", [8, 72, 136, 264])
+@pytest.mark.parametrize("T,N", [(5, 16), (7000, 16), (5, 30), (4100, 30), (4100, 32), (5, 64),
+                                 (1600, 64), (5, 80), (1300, 80), (500, 256)])
+@pytest.mark.parametrize("wd", [torch.float32, torch.bfloat16])
+def test_rows_behind_w_are_not_read(gpu, T, N, D, wd):
+    """W as the front of a larger buffer: what lies behind its last row (NaN, or
+    zeros) makes no difference, also where d_model ends inside a chunk."""
+    print(f"router W tail T{T} N{N} D{D} {wd}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(T + N + D)
+    x = torch.randn(T, D, generator=g).to(gpu, torch.bfloat16)
+    w = torch.randn(D, N, generator=g).mul(0.1)
+    got = []
+    for behind in (0.0, float("nan")):
+        buf = torch.full(((D + 256) * N,), behind, dtype=wd, device=gpu)
+        buf[:D * N] = w.to(gpu, wd).reshape(-1)
+        got.append(K.router(x, buf[:D * N].view(D, N), None, min(4, N), _lib.ROUTE_SOFTMAX, 1.0))
+    torch.cuda.synchronize()
+    assert torch.isfinite(got[0][0]).all()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
