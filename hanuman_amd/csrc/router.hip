@@ -387,11 +387,8 @@ __device__ __forceinline__ void barrier_lds_only() {
 // MFMA steps (of 4 d) per chunk.  Short chains (4 tokens) take 64 where the
 // registers allow two chunks of W (32 took 19.4 instead of 16.9 us at one
 // token, 64 experts, d_model 2048); 16-token ones 32, whose registers let more
-// workgroups share a CU (16384 tokens: 83 against 91 us), 16 where the
-// workgroup's x would not fit 64 KB.
-constexpr int router_steps(int mt, int tok) {
-  return tok == 4 ? (mt <= 8 ? 64 : 32) : (mt == 1 ? 16 : 32);
-}
+// workgroups share a CU (16384 tokens: 83 against 91 us).
+constexpr int router_steps(int mt, int tok) { return tok == 4 && mt <= 8 ? 64 : 32; }
 
 // Waves per expert tile, each with tokens of its own: a workgroup has at least
 // four waves, one per SIMD (two-wave workgroups two to a CU shared SIMDs: 79
@@ -657,26 +654,34 @@ __global__ __launch_bounds__(64 * MT * router_groups(MT), MT > 8 || TOK == 16 ? 
   }
 }
 
-// Two expert tiles (17..32 experts) and more tokens than short chains fill the
-// chip with: x and W staged in LDS as float32 through registers two chunks
-// ahead, each wave (one chain) widening both operands.  Here W's rows are so
-// short that the direct loads of router_kernel are mostly address work, and
-// half of the waves would load the same ones: at 8192 tokens, 32 experts,
-// d_model 4096 with x's quantisation this form takes 59.5 us, that one 69.9
-// (62.6 alone).  W is 16-byte aligned and n_experts a multiple of the W
-// elements in 16 bytes, so a chunk of W is staged with 16-byte loads.
+// NT = 1 or 2 expert tiles and more tokens than short chains fill the chip
+// with: x and W staged in LDS as float32 through registers two chunks ahead,
+// each wave (one chain) widening both operands.  Here W's rows are so short that
+// the direct loads of router_kernel are mostly address work, and several waves
+// would load the same ones.  This form against that one, us: 8192 tokens, d_model
+// 4096, 32 experts with x's quantisation 59.5 / 69.9 (59.5 / 62.6 alone); d_model
+// 2048, 8 experts 36.3 / 47.0, 16384 tokens 37.1 / 48.0; 16 experts, d_model 1024,
+// 22.1 / 27.3 (40000 tokens 63.1 / 60.3, the one measured loss); 10 experts (by
+// elements), 40000 tokens, d_model 2048 86 / 107.
+//
+// WV: W is 16-byte aligned and n_experts a multiple of the W elements in 16
+// bytes, so a chunk of W is staged with 16-byte loads; else (one tile only: 18
+// and 30 experts gain nothing) by elements, in chunks of half the length, whose
+// registers would spill.
 template <int V>
 struct IntC {
   static constexpr int value = V;
 };
 
+template <int NT, bool WV>
 struct alignas(16) RouterStagedLds {
-  static constexpr int kDc = 128;  // d per chunk (one barrier per chunk)
-  float x[2][32][kDc + 4];         // 16-byte aligned rows
-  float w[2][kDc][32 + 8];
+  static constexpr int kDc = WV ? 128 : 64;  // d per chunk (one barrier per chunk)
+  static constexpr int kTB = 64 / NT;        // tokens
+  float x[2][kTB][kDc + 4];                  // 16-byte aligned rows
+  float w[2][kDc][16 * NT + 8];
 };
 
-template <typename XT, typename WT, bool QX>
+template <int NT, bool WV, typename XT, typename WT, bool QX>
 __global__ __launch_bounds__(256) void router_staged_kernel(
     const XT* __restrict__ x, const WT* __restrict__ w, const float* __restrict__ bias,
     int64_t tokens, int d_model, int n_experts, int top_k, int mode, float rsf,
@@ -690,17 +695,19 @@ __global__ __launch_bounds__(256) void router_staged_kernel(
     }
   }
   constexpr int kThr = 256;
-  constexpr int kNP = 32;                                     // two expert tiles
-  constexpr int kTB = 32;                                     // two token groups
-  constexpr int kDc = RouterStagedLds::kDc;
+  constexpr int kNP = 16 * NT;
+  constexpr int kTB = RouterStagedLds<NT, WV>::kTB;
+  constexpr int kTG = kTB / 16;                               // token groups
+  constexpr int kDc = RouterStagedLds<NT, WV>::kDc;
   constexpr int kE16 = 16 / static_cast<int>(sizeof(WT));     // W elements per 16-byte load
   constexpr int kWV = kDc * kNP / kE16 / kThr;                // 16-byte W loads per thread per chunk
-  __shared__ RouterStagedLds lds;
+  constexpr int kWPer = kDc * kNP / kThr;                     // W elements per thread per chunk
+  __shared__ RouterStagedLds<NT, WV> lds;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int tg = wave & 1;
-  const int ep = wave >> 1;
+  const int tg = wave % kTG;
+  const int ep = wave / kTG;
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kTB;
 
   // Staging assignment: x elements (tt, dd..dd+7) = (g / kXT, (g % kXT) * 8) for
@@ -725,7 +732,14 @@ __global__ __launch_bounds__(256) void router_staged_kernel(
   // Two register sets: the loads of chunk c + 2 are issued at the start of
   // chunk c, so a load has two chunks of MFMAs to arrive before it is parked.
   X8<XT> xr0[kXR], xr1[kXR];
-  uint32_t wr0[4 * kWV], wr1[4 * kWV];
+  constexpr int kWRegs = WV ? 4 * kWV : kWPer;
+  uint32_t wr0[kWRegs], wr1[kWRegs];
+  // Element q of the staging by elements: row idx / kNP, expert idx % kNP, idx =
+  // q * kThr + tid.
+  auto w_ok = [&](int q, int d0) __attribute__((always_inline)) {
+    const int idx = q * kThr + tid;
+    return idx % kNP < n_experts && d0 + idx / kNP < d_model;
+  };
   // Vector q covers elements idx .. idx + kE16 - 1 (idx = (q*kThr + tid) *
   // kE16) of the chunk, i.e. row idx / n_experts, experts idx % n_experts ...
   auto wv_idx = [&](int q) __attribute__((always_inline)) { return (q * kThr + tid) * kE16; };
@@ -735,14 +749,27 @@ __global__ __launch_bounds__(256) void router_staged_kernel(
       const int dx = d0 + xs_dd[r];
       xr[r].load(x + xs_row[r] + (dx < d_model ? dx : 0));
     }
+    if constexpr (WV) {
 #pragma unroll
-    for (int q = 0; q < kWV; ++q) {
-      const int idx = wv_idx(q);
-      const bool ok = idx < kDc * n_experts && d0 + idx / n_experts < d_model;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(
-          w + (ok ? static_cast<int64_t>(d0) * n_experts + idx : 0));
+      for (int q = 0; q < kWV; ++q) {
+        const int idx = wv_idx(q);
+        const bool ok = idx < kDc * n_experts && d0 + idx / n_experts < d_model;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(
+            w + (ok ? static_cast<int64_t>(d0) * n_experts + idx : 0));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wr[4 * q + j] = v[j];
+        for (int j = 0; j < 4; ++j) wr[4 * q + j] = v[j];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < kWPer; ++q) {
+        const int idx = q * kThr + tid;
+        const int64_t off = static_cast<int64_t>(d0 + idx / kNP) * n_experts + idx % kNP;
+        const WT v = w[w_ok(q, d0) ? off : 0];
+        if constexpr (sizeof(WT) == 4)
+          wr[q] = __float_as_uint(v);
+        else
+          wr[q] = static_cast<uint32_t>(v) << 16;
+      }
     }
     // Keep the loads ahead of the MFMAs; the masking happens in park().
     __builtin_amdgcn_sched_barrier(0);
@@ -760,36 +787,44 @@ __global__ __launch_bounds__(256) void router_staged_kernel(
       *reinterpret_cast<f32x4*>(&lds.x[buf][xs_tt[r]][xs_dd[r]]) = lo;
       *reinterpret_cast<f32x4*>(&lds.x[buf][xs_tt[r]][xs_dd[r] + 4]) = hi;
     }
+    if constexpr (WV) {
 #pragma unroll
-    for (int q = 0; q < kWV; ++q) {
-      const int idx = wv_idx(q);
-      if (idx < kDc * n_experts) {
-        const int d = idx / n_experts;
-        const int n = idx - d * n_experts;
-        const bool ok = d0 + d < d_model;
-        float* dst = &lds.w[buf][d][n];
-        if (sizeof(WT) == 4) {
-          f32x4 v;
+      for (int q = 0; q < kWV; ++q) {
+        const int idx = wv_idx(q);
+        if (idx < kDc * n_experts) {
+          const int d = idx / n_experts;
+          const int n = idx - d * n_experts;
+          const bool ok = d0 + d < d_model;
+          float* dst = &lds.w[buf][d][n];
+          if (sizeof(WT) == 4) {
+            f32x4 v;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = ok ? __uint_as_float(wr[4 * q + j]) : 0.0f;
-          *reinterpret_cast<f32x4*>(dst) = v;
-        } else {
-          f32x4 lo, hi;
+            for (int j = 0; j < 4; ++j) v[j] = ok ? __uint_as_float(wr[4 * q + j]) : 0.0f;
+            *reinterpret_cast<f32x4*>(dst) = v;
+          } else {
+            f32x4 lo, hi;
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const uint32_t a = wr[4 * q + j], b = wr[4 * q + 2 + j];
-            lo[2 * j] = ok ? __uint_as_float(a << 16) : 0.0f;
-            lo[2 * j + 1] = ok ? __uint_as_float(a & 0xffff0000u) : 0.0f;
-            hi[2 * j] = ok ? __uint_as_float(b << 16) : 0.0f;
-            hi[2 * j + 1] = ok ? __uint_as_float(b & 0xffff0000u) : 0.0f;
+            for (int j = 0; j < 2; ++j) {
+              const uint32_t a = wr[4 * q + j], b = wr[4 * q + 2 + j];
+              lo[2 * j] = ok ? __uint_as_float(a << 16) : 0.0f;
+              lo[2 * j + 1] = ok ? __uint_as_float(a & 0xffff0000u) : 0.0f;
+              hi[2 * j] = ok ? __uint_as_float(b << 16) : 0.0f;
+              hi[2 * j + 1] = ok ? __uint_as_float(b & 0xffff0000u) : 0.0f;
+            }
+            *reinterpret_cast<f32x4*>(dst) = lo;
+            *reinterpret_cast<f32x4*>(dst + 4) = hi;
           }
-          *reinterpret_cast<f32x4*>(dst) = lo;
-          *reinterpret_cast<f32x4*>(dst + 4) = hi;
         }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < kWPer; ++q) {
+        const int idx = q * kThr + tid;
+        lds.w[buf][idx / kNP][idx % kNP] = w_ok(q, d0) ? __uint_as_float(wr[q]) : 0.0f;
       }
     }
   };
-  if (n_experts < kNP) {
+  if (WV && n_experts < kNP) {
     // Expert columns past n_experts are never written by the vector staging:
     // zero them once in both buffers.
     for (int i = tid; i < 2 * kDc * kNP; i += kThr) {
@@ -946,15 +981,15 @@ void launch_router_tok(const void* x, const void* w, const float* bias, int64_t 
                      logits, top_idx, gates, nullptr, nullptr, rblocks);
 }
 
-template <typename XT, typename WT>
+template <int NT, bool WV, typename XT, typename WT>
 void launch_router_staged(const void* x, const void* w, const float* bias, int64_t tokens,
                           int d_model, int n_experts, int top_k, int mode, float rsf,
                           float* logits, int32_t* top_idx, float* gates, hipStream_t stream,
                           XQuant xq) {
-  const int rblocks = static_cast<int>(ceil_div(tokens, 32));
+  const int rblocks = static_cast<int>(ceil_div(tokens, RouterStagedLds<NT, WV>::kTB));
   if constexpr (sizeof(XT) == 2) {
     if (xq.q != nullptr) {
-      hipLaunchKernelGGL((router_staged_kernel<XT, WT, true>),
+      hipLaunchKernelGGL((router_staged_kernel<NT, WV, XT, WT, true>),
                          dim3(static_cast<unsigned>(rblocks + ceil_div(tokens, 4))), dim3(256), 0,
                          stream, static_cast<const XT*>(x), static_cast<const WT*>(w), bias, tokens,
                          d_model, n_experts, top_k, mode, rsf, logits, top_idx, gates, xq.q,
@@ -962,7 +997,7 @@ void launch_router_staged(const void* x, const void* w, const float* bias, int64
       return;
     }
   }
-  hipLaunchKernelGGL((router_staged_kernel<XT, WT, false>), dim3(static_cast<unsigned>(rblocks)),
+  hipLaunchKernelGGL((router_staged_kernel<NT, WV, XT, WT, false>), dim3(static_cast<unsigned>(rblocks)),
                      dim3(256), 0, stream, static_cast<const XT*>(x), static_cast<const WT*>(w),
                      bias, tokens, d_model, n_experts, top_k, mode, rsf, logits, top_idx, gates,
                      nullptr, nullptr, rblocks);
@@ -984,19 +1019,25 @@ void launch_router(const void* x, const void* w, const float* bias, int64_t toke
                                             logits, top_idx, gates, stream, xq);
     return;
   }
-  if constexpr (MT == 2) {
-    if (n_experts % (16 / static_cast<int>(sizeof(WT))) == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0) {
-      launch_router_staged<XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf, logits,
-                                   top_idx, gates, stream, xq);
+  const bool wv = n_experts % (16 / static_cast<int>(sizeof(WT))) == 0 &&
+                  reinterpret_cast<uintptr_t>(w) % 16 == 0;
+  if constexpr (MT <= 2) {
+    if (wv) {
+      launch_router_staged<MT, true, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
+                                             logits, top_idx, gates, stream, xq);
       return;
     }
   }
-  if (d_model % (4 * router_steps(MT, 16)) == 0)
+  if constexpr (MT == 1) {
+    launch_router_staged<1, false, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
+                                           logits, top_idx, gates, stream, xq);
+  } else if (d_model % (4 * router_steps(MT, 16)) == 0) {
     launch_router_tok<MT, 16, false, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
                                              logits, top_idx, gates, stream, xq);
-  else
+  } else {
     launch_router_tok<MT, 16, true, XT, WT>(x, w, bias, tokens, d_model, n_experts, top_k, mode, rsf,
                                             logits, top_idx, gates, stream, xq);
+  }
 }
 
 template <int MT>

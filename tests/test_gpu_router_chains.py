@@ -17,6 +17,10 @@ CASES = [
     (1, 8, 1, 1, "bf16", "f32"),          # one chunk, two MFMA steps, one expert
     (3, 264, 16, 4, "f32", "bf16"),       # one tile, chunk tail of 8 (256 + 8)
     (5, 520, 17, 5, "bf16", "f32"),       # two tiles, one lane of the second
+    (6144, 136, 16, 4, "bf16", "f32"),    # last token count of the short chains at one tile
+    (6145, 136, 16, 4, "bf16", "f32"),    # and the first past it (staged W)
+    (6151, 72, 12, 3, "f32", "bf16"),     # W staged by elements (12 % 8), chunk tail of 8 (64 + 8)
+    (6200, 264, 7, 2, "bf16", "f32"),
     (4093, 72, 30, 3, "bf16", "bf16"),    # two tiles, 16-token chains, W staged off (30 % 8)
     (3072, 136, 32, 4, "bf16", "f32"),    # last token count of the short chains at two tiles
     (3073, 136, 32, 4, "bf16", "f32"),    # and the first past it (staged W)
@@ -56,6 +60,21 @@ def test_router_chains_bit_exact(gpu, case):
     for name, got, ref in (("logits", logits, logits_ref), ("gates", g, g_ref)):
         assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.view(np.uint32)), name
     assert np.array_equal(idx.cpu().numpy(), idx_ref)
+
+
+@pytest.mark.parametrize("T,N", [(6145, 16), (6151, 12), (3073, 32), (1537, 64)])
+def test_router_with_quantisation_past_the_switch(gpu, T, N):
+    """The launch that quantises x beside the router, in the forms for many
+    tokens, against the two separate launches."""
+    print(f"router quant T{T} N{N}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(T)
+    x = torch.randn(T, 264, generator=g).to(gpu, torch.bfloat16)
+    w = torch.randn(264, N, generator=g).mul(0.1).to(gpu, torch.bfloat16)
+    got = K.router_quant_fp8(x, w, None, 4, _lib.ROUTE_SOFTMAX, 1.0)
+    ref = (*K.router(x, w, None, 4, _lib.ROUTE_SOFTMAX, 1.0), *K.quantize_rows_fp8(x))
+    torch.cuda.synchronize()
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("D", [8, 72, 136, 264])
