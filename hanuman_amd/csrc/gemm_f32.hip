@@ -229,19 +229,27 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_kernel(
   }
 }
 
-__global__ __launch_bounds__(256) void grouped_wgrad_f32_kernel(
-    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
-    const int32_t* __restrict__ offsets, int mdim, int ncols, int nsplit, float* __restrict__ C0,
-    float* __restrict__ C1) {
-  __shared__ float sa[kF32K][kF32Tile + 1];
-  __shared__ float sb[kF32K][kF32Tile + 1];
+struct WgradTile {
+  int e, m0, n0;
+};
+// S x S tile t of the experts' [mdim][ncols] gradients.
+template <int S>
+__device__ __forceinline__ WgradTile wgrad_f32_tile(int t, int mdim, int ncols) {
+  const int tm = mdim / S, tn = ncols / S;
+  const int e = t / (tm * tn);
+  const int rem = t - e * tm * tn;
+  return {e, (rem / tn) * S, (rem - (rem / tn) * tn) * S};
+}
+
+// The 64 x 64 tile at (m0, n0) of expert e, summed over the rows r_lo .. r_hi.
+__device__ __forceinline__ void wgrad_f32_sum(float (&sa)[kF32K][kF32Tile + 1],
+                                              float (&sb)[kF32K][kF32Tile + 1],
+                                              const float* __restrict__ A, int64_t lda,
+                                              const float* __restrict__ B, int64_t ldb, int e, int m0,
+                                              int n0, int64_t r_lo, int64_t r_hi, int mdim, int ncols,
+                                              int nsplit, float* __restrict__ C0,
+                                              float* __restrict__ C1) {
   const int tid = threadIdx.x;
-  const int tm = mdim / kF32Tile, tn = ncols / kF32Tile;
-  const int e = static_cast<int>(blockIdx.x / (tm * tn));
-  const int rem = static_cast<int>(blockIdx.x - static_cast<int64_t>(e) * tm * tn);
-  const int m0 = (rem / tn) * kF32Tile;
-  const int n0 = (rem - (rem / tn) * tn) * kF32Tile;
-  const int64_t r_lo = offsets[e], r_hi = offsets[e + 1];
   const int lr = tid >> 4, lc = (tid & 15) * 4;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -286,6 +294,17 @@ __global__ __launch_bounds__(256) void grouped_wgrad_f32_kernel(
   }
 }
 
+__global__ __launch_bounds__(256) void grouped_wgrad_f32_kernel(
+    const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
+    const int32_t* __restrict__ offsets, int mdim, int ncols, int nsplit, float* __restrict__ C0,
+    float* __restrict__ C1) {
+  __shared__ float sa[kF32K][kF32Tile + 1];
+  __shared__ float sb[kF32K][kF32Tile + 1];
+  const WgradTile t = wgrad_f32_tile<kF32Tile>(static_cast<int>(blockIdx.x), mdim, ncols);
+  wgrad_f32_sum(sa, sb, A, lda, B, ldb, t.e, t.m0, t.n0, offsets[t.e], offsets[t.e + 1], mdim, ncols,
+                nsplit, C0, C1);
+}
+
 // ---- few tiles: K split over the waves ----------------------------------------
 // Where 64 x 64 tiles are fewer than the CUs (a short prompt, one shared expert,
 // a weight gradient of few experts), the kernels above are bound by the latency
@@ -304,6 +323,12 @@ __global__ __launch_bounds__(256) void grouped_wgrad_f32_kernel(
 // (256 tiles) and 32.2 -> 27.8 (512).  Past the lines below the operands' traffic
 // (twice that of a 64 x 64 tile) loses: gate/up of 2048 rows 17.1 against 22.4
 // (256 tiles), 16 experts' weight gradients (1536 tiles) 30.2 against 38.8.
+// Short sums lose too, for their four times as many workgroups: a segment's
+// weight gradient gains from about 40 rows up where these are one round over the
+// chip (128 tiles, 32 rows 3.9 against 3.6, 128 rows 6.7 / 4.4), 120 where they
+// are two (256 tiles, 32 rows 4.1 / 5.5, 128 rows 6.9 / 6.6, 256 rows 10.8 / 11.0,
+// 512 rows 25 / 17) and 360 for three (512 tiles, 96 rows 8.3 / 11.0, 512 rows
+// 31 / 27).
 constexpr int kF32Split = 32;
 
 // A lane's f32x4 groups of the four waves' partial fragments, added in wave
@@ -493,19 +518,34 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_split_kernel(
   *reinterpret_cast<f32x4*>(C + row * ldc + col) = v;
 }
 
+// Four workgroups a 64 x 64 tile.  The lengths of the segments are known only
+// here: one of fewer than min_rows is summed as above, by the first quarter of
+// the workgroups, beside their parts of the others.
 __global__ __launch_bounds__(256) void grouped_wgrad_f32_split_kernel(
     const float* __restrict__ A, int64_t lda, const float* __restrict__ B, int64_t ldb,
-    const int32_t* __restrict__ offsets, int mdim, int ncols, int nsplit, float* __restrict__ C0,
-    float* __restrict__ C1) {
-  __shared__ f32x4 part[4 * 4 * 64];
+    const int32_t* __restrict__ offsets, int mdim, int ncols, int nsplit, int min_rows,
+    float* __restrict__ C0, float* __restrict__ C1) {
+  union Lds {
+    f32x4 part[4 * 4 * 64];
+    float ab[2][kF32K][kF32Tile + 1];
+  };
+  __shared__ Lds lds;
+  f32x4* const part = lds.part;
   const int tid = threadIdx.x;
-  const int tm = mdim / kF32Split, tn = ncols / kF32Split;
-  const int e = static_cast<int>(blockIdx.x / (tm * tn));
-  const int rem = static_cast<int>(blockIdx.x - static_cast<int64_t>(e) * tm * tn);
-  const int m0 = (rem / tn) * kF32Split;
-  const int n0 = (rem - (rem / tn) * tn) * kF32Split;
+  const WgradTile t = wgrad_f32_tile<kF32Split>(static_cast<int>(blockIdx.x), mdim, ncols);
+  const int e = t.e, m0 = t.m0, n0 = t.n0;
   const int64_t r_lo = __builtin_amdgcn_readfirstlane(offsets[e]);
   const int rows = __builtin_amdgcn_readfirstlane(offsets[e + 1]) - static_cast<int>(r_lo);
+  if (blockIdx.x < gridDim.x / 4) {
+    const WgradTile w = wgrad_f32_tile<kF32Tile>(static_cast<int>(blockIdx.x), mdim, ncols);
+    const int64_t r0 = offsets[w.e], r1 = offsets[w.e + 1];
+    if (r1 - r0 < min_rows) {
+      wgrad_f32_sum(lds.ab[0], lds.ab[1], A, lda, B, ldb, w.e, w.m0, w.n0, r0, r1, mdim, ncols, nsplit,
+                    C0, C1);
+      __syncthreads();
+    }
+  }
+  if (rows < min_rows) return;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hi2 = lane >> 5;
   // One chunk of 32 rows: MFMA s takes rows 2 s + hi2.  The resources start at
@@ -605,9 +645,14 @@ int launch_wgrad_f32(const float* A, int64_t lda, const float* B, int64_t ldb,
                      float* C0, float* C1, hipStream_t s, const char* what) {
   const int64_t grid = static_cast<int64_t>(n_experts) * (mdim / kF32Tile) * (ncols / kF32Tile);
   HMOE_REQUIRE(grid < (int64_t(1) << 31), "%s: too many tiles", what);
-  if (grid <= int64_t(2) * f32_cus(s)) {
+  const int64_t cus = f32_cus(s);
+  if (grid <= 2 * cus) {
+    // Three workgroups fit a CU (their registers): the more rounds of them, the
+    // longer a sum has to be to gain, see above.
+    const int64_t rounds = ceil_div(4 * grid, 3 * cus);
+    const int min_rows = rounds == 1 ? 40 : rounds == 2 ? 120 : 360;
     hipLaunchKernelGGL(grouped_wgrad_f32_split_kernel, dim3(static_cast<unsigned>(4 * grid)), dim3(256),
-                       0, s, A, lda, B, ldb, offsets, mdim, ncols, nsplit, C0, C1);
+                       0, s, A, lda, B, ldb, offsets, mdim, ncols, nsplit, min_rows, C0, C1);
     return check_launch(what);
   }
   hipLaunchKernelGGL(grouped_wgrad_f32_kernel, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, A,

@@ -15,7 +15,21 @@ CASES = [
     ([771], 512, 768),          # gate/up split (156 tiles of 64 x 64)
     ([2048], 256, 512),         # gate/up not (256 tiles), down split
     ([513, 511, 0, 1024, 40, 1, 900, 1107], 256, 512),
+    # weight gradients: segments either side of the length from which a sum is
+    # split, 40, 120 and 360 rows for one, two and three rounds of workgroups
+    ([39, 0, 40, 41], 64, 128),
+    ([119, 120, 0, 121, 1, 359, 360, 361], 256, 512),
+    # and more 64 x 64 tiles (1536, 3072) than two a CU: never split
+    ([37, 0, 64, 65, 1, 16, 100, 17, 31, 48, 2, 80, 15, 128, 33, 3], 512, 768),
 ]
+
+
+def test_weight_gradient_cases_take_both_kernels(gpu):
+    """The two sides of the switch at two 64 x 64 tiles a CU."""
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    tiles = [[len(lens) * (D // 64) * (f // 64) for f in (F, 2 * F)] for lens, D, F in CASES]
+    assert max(tiles[-2]) <= 2 * cus < min(tiles[-1])
+    assert [-(-4 * t // (3 * cus)) for t in tiles[-3] + tiles[-2]] == [1, 1, 2, 3]
 
 
 @pytest.mark.parametrize("lens,D,F", CASES, ids=lambda v: str(v).replace(" ", ""))
