@@ -314,7 +314,11 @@ constexpr int64_t kFusedScanEntries = 65536;
 
 // SELF: plans of at most kSelfHistRows slots count the whole top_idx in every
 // workgroup instead (8 loads in flight a thread, LDS atomics on exact integers),
-// so the plan is one launch.
+// so the plan is one launch.  Each slot is counted once, before or from this
+// block on, in one of up to 16 arrays (one more for every 512 slots) that
+// neighbouring lanes share: with one array, 4096 tokens that all take the same 2
+// of 16 experts queued up at their counters for 11.7 us, against 8.0 for the two
+// launches and 7.5 with 16 (8192 tokens on one expert: 18.8, 8.7 and 9.7).
 constexpr int64_t kSelfHistRows = 8192;
 
 template <bool SELF>
@@ -353,13 +357,16 @@ __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
   // tid taking experts tid, tid + 256, ... when N > 256); group g sums the
   // blocks g, g + G, ..., so the 64 lanes of a wave read 64 consecutive
   // experts of one block.
-  const int G = SELF || n_experts >= kPlanThreads ? 1 : kPlanThreads / n_experts;
+  int G = n_experts >= kPlanThreads ? 1 : kPlanThreads / n_experts;
   if constexpr (SELF) {
-    for (int e = tid; e < n_experts; e += kPlanThreads) {
-      part_pre[e] = 0;
-      part_tot[e] = 0;
+    G = 1;
+    while (G < 16 && 2 * G * n_experts <= kMaxExperts && 1024 * G <= rows) G *= 2;
+    for (int i = tid; i < G * n_experts; i += kPlanThreads) {
+      part_pre[i] = 0;
+      part_tot[i] = 0;
     }
     __syncthreads();
+    const int copy = (tid & (G - 1)) * n_experts;
     const int n = static_cast<int>(rows), before = static_cast<int>(blk_base);
     for (int i0 = tid; i0 < n; i0 += 8 * kPlanThreads) {
       int v[8];
@@ -372,8 +379,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
       for (int u = 0; u < 8; ++u) {
         const int i = i0 + u * kPlanThreads;
         if (i < n && static_cast<unsigned>(v[u]) < static_cast<unsigned>(n_experts)) {
-          atomicAdd(&part_tot[v[u]], 1);
-          if (i < before) atomicAdd(&part_pre[v[u]], 1);
+          atomicAdd(i < before ? &part_pre[copy + v[u]] : &part_tot[copy + v[u]], 1);
         }
       }
     }
@@ -386,9 +392,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
       // eight loads in flight at a time (the sums are exact integer sums)
       for (; bb + 7 * G < nblk; bb += 8 * G) {
         int32_t c[8];
-  #pragma unroll
+#pragma unroll
         for (int u = 0; u < 8; ++u) c[u] = hist[static_cast<int64_t>(bb + u * G) * n_experts + e];
-  #pragma unroll
+#pragma unroll
         for (int u = 0; u < 8; ++u) {
           tot += c[u];
           if (bb + u * G < b) pre += c[u];
@@ -411,6 +417,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_rank_fused_kernel(
       pre += part_pre[g * n_experts + e];
       tot += part_tot[g * n_experts + e];
     }
+    if (SELF) tot += pre;  // counted from this block on
     if (b == 0) counts[e] = tot;
     // per-wave bases of this block's four waves
     int32_t run = pre;
@@ -690,7 +697,7 @@ int launch_plan(const int32_t* top_idx, int64_t tokens, int top_k, int n_experts
   const int64_t rows = tokens * top_k;
   const int64_t rows_cap = hmoe_rows_cap(tokens, top_k, n_experts, capacity);
   const int nblk = static_cast<int>(plan_blocks(rows));
-  // (few experts' counters in one workgroup serialise its atomics: from 8 up)
+  // (the atomics of fewer than 8 experts' counters would queue up)
   if (rows > 0 && (rows <= kSlotsPerBlock || (rows <= kSelfHistRows && n_experts >= 8))) {
     hipLaunchKernelGGL(plan_rank_fused_kernel<true>, dim3(nblk), dim3(kPlanThreads), 0, s, top_idx,
                        rows, n_experts, capacity, static_cast<const int32_t*>(nullptr), nblk, counts,

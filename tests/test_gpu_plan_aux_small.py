@@ -10,6 +10,21 @@ from hanuman_amd import kernels as K
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("T,Kk,N,cap", [(1, 1, 9, 1), (512, 2, 16, 700), (600, 3, 64, 5000),
+                                        (4096, 2, 16, 3000), (8192, 1, 64, 8192), (1023, 8, 100, 900)])
+def test_plan_one_launch_collapsed_load(gpu, T, Kk, N, cap):
+    """Every token on the same experts, at each number of counter arrays (1 to 16)."""
+    print(f"plan collapsed {T} {Kk} {N}", flush=True)
+    idx = np.tile(np.arange(N - Kk, N, dtype=np.int32), (T, 1))
+    ref = O.dispatch_plan(idx, N, cap)
+    plan = K.dispatch_plan(torch.from_numpy(idx).to(gpu), N, cap)
+    torch.cuda.synchronize()
+    for name in ("counts", "offsets", "slot_pos"):
+        assert np.array_equal(getattr(plan, name).cpu().numpy(), ref[name]), name
+    kept = int(ref["offsets"][-1])
+    assert np.array_equal(plan.perm_src.cpu().numpy()[:kept], ref["perm_src"][:kept])
+
+
 @pytest.mark.parametrize("T,Kk,N,cap", [(1, 1, 1, 1), (512, 2, 7, 130), (513, 2, 7, 130),
                                         (1024, 8, 8, 900), (1025, 8, 8, 900), (2730, 3, 300, 20)])
 def test_plan_one_launch_matches_oracle(gpu, T, Kk, N, cap):
