@@ -53,6 +53,7 @@ SIGNATURES = {
     "hmoe_grouped_gate_up_gather": (_i32, [_vp, _i64, _i32, _vp, _vp, _i32, _i64, _i32, _i32, _vp,
                                            _vp, _vp]),
     "hmoe_grouped_down": (_i32, [_vp, _vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp]),
+    "hmoe_grouped_tile": (_i32, [_i64, _i32, _i64, _i32, _i32, _vp, _vp]),
     "hmoe_grouped_shared_joins": (_i32, [_i64, _i32, _i64, _i32, _i32, _i32, _vp]),
     "hmoe_grouped_gate_up_gather_shared": (_i32, [_vp, _i64, _i32, _vp, _vp, _i32, _i64, _i32,
                                                   _i32, _vp, _vp, _i32, _vp, _vp]),

@@ -2487,17 +2487,31 @@ int allow_dynamic_lds(int dev) {
   return HMOE_OK;
 }
 
+// The row tiles of an expert of `mean` rows on average, rounded up expert by
+// expert: the counts, which only the device knows, are taken to spread as chance
+// has it (normal, variance = mean), and where a tile more is likely the
+// half tile that this rounding costs is counted in full.
+double row_tiles(double mean, double sd, int bm) {
+  const double near = 4.0 * sd;
+  if (mean + near <= bm) return 1.0;
+  if (mean > 6.0 * bm) return mean / bm + 0.5;
+  double tiles = 1.0 + std::max(0, static_cast<int>((mean - near) / bm));
+  for (double k = tiles; k * bm < mean + near; k += 1.0)
+    tiles += 0.5 * std::erfc((k * bm + 0.5 - mean) / (sd * 1.4142135623730951));
+  return mean + 1.5 * sd <= bm ? tiles : std::max(tiles, mean / bm + 0.5);
+}
+
 // The tile of a grouped GEMM over `rows` rows on n_experts experts: 256 x 256
 // (grouped_gemm_regs, grouped_gemm_w8_fp8) or one of grouped_gemm_few's, by the
-// smallest estimated time.  With the rows spread evenly (the counts are on the
-// device) an expert has mean +- sqrt(mean) of them, so its row tiles are one
-// while mean + 1.5 sqrt(mean) rows fit, else about mean / bm + 1/2.  A round of
-// tiles over the CUs takes the tile's operand bytes at the 20 B/clk a CU draws
-// from L2 plus ~2 us; in units of 128 bytes (2.67 ns) that is ks (bm + bn) +
-// 750.  No shape is faster than streaming the touched experts' weights (5.5
+// smallest estimated time.  A round of tiles over the CUs takes the tile's
+// operand bytes at the 20 B/clk a CU draws from L2 plus ~2 us; in units of 128
+// bytes (2.67 ns) that is ks (bm + bn) + 750, and row_tiles says how many
+// there are (less a quarter of one: a tile that is not likely opens no round).
+// No shape is faster than streaming the touched experts' weights (5.5
 // TB/s at best; few-rows tiles reach 1.15 times that time, the 256 x 256 ones
 // 1.4).  Between shapes at that floor, 128 columns are best for long K (32
-// steps and more) and 256 for short.  Measured (old = 256 x 256), us:
+// steps and more) and 256 for short, and 256 x 256 where it is within 3%.
+// Measured (old = 256 x 256), us:
 //   gate/up 64 experts, D 2048, F 1024: 1 token, top-8, old 47.2, 32 x 64 19.0;
 //     48 tokens 148.9, 32 x 128 114.9; 768 tokens 146.5, 128 x 128 128.3;
 //   down, same layer: 27.3 -> 10.9, 58.3 -> 42.4, 68.7 -> 57.2;
@@ -2506,8 +2520,16 @@ int allow_dynamic_lds(int dev) {
 //   one segment, D 1536, F 768: 333 rows 35.9 -> 13.2 (64 x 64), 4096 rows
 //     39.6 -> 31.3 (128 x 256); 16384 rows, D 2048, F 1024 121.5 against 144.7;
 //   e4m3, 32 experts, D 4096, F 2048, top-4: 100 tokens 142.8 -> 115.3 and 56.5
-//     -> 42.7; 1600 tokens 159.9 against 172.9: old.
-//
+//     -> 42.7; 1600 tokens 159.9 against 172.9: old;
+//   more than one 128-row tile an expert, gate/up: 80 experts of 140 rows 106.5
+//     against 146.6 (128 x 256), D 4096, F 2048 32 experts of 190 rows 285 / 368,
+//     D 1024, F 2048 16 of 125 rows 38.3 / 52.4: old.
+// Over 12 layer shapes, 1 to 1000 rows an expert and seven GEMMs of each, the
+// tile taken is 1.01 times the fastest shape's time on average, and 1.06 where the
+// experts' popularity falls as 1 / rank (64 experts of 125 rows on average, 37 to
+// 1000: gate/up 187 -> 154).  What loses is a load that is on few experts
+// altogether, which the host cannot see: all of 1000 tokens on the same 8 of 80
+// experts, gate/up 47 -> 70.
 //
 // Dense groups (in a launch of the few-rows kernel only) add their tiles and
 // their weights; the few tiles past whole rounds then matter, so there full
@@ -2516,7 +2538,7 @@ int allow_dynamic_lds(int dev) {
 void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int cus, int* bm, int* bn,
                  int dense_groups = 0, int64_t dense_rows = 0, double* units = nullptr) {
   const double n_eff = rows < n_experts ? static_cast<double>(rows) : n_experts;
-  const double mean = rows / n_eff;
+  const double mean = rows / n_eff, sd = std::sqrt(mean);
   const double ks = row_bytes / 128.0;
   const double floor = (n_eff + dense_groups) * ncols * ks / (5.5e6 / 128.0) / 0.002667;
   static const int kShapes[][2] = {{256, 256}, {128, 256}, {128, 128}, {64, 256}, {64, 128},
@@ -2527,16 +2549,12 @@ void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int 
     if (dense_groups > 0) {
       // weights read twice for a second row tile measured slower than 128 rows
       // (layer of 64 experts, D 2048, F 1024, 640 tokens: 287 us against 263)
-      if (old || (sh[0] < 128 && n_eff > 1.0 && mean + std::sqrt(mean) > sh[0])) continue;
+      if (old || (sh[0] < 128 && n_eff > 1.0 && mean + sd > sh[0])) continue;
     }
-    double mt;
-    if (n_experts == 1)
-      mt = std::ceil(mean / sh[0]);
-    else
-      mt = n_eff * (mean + 1.5 * std::sqrt(mean) <= sh[0] ? 1.0 : mean / sh[0] + 0.5);
+    const double mt = n_experts == 1 ? std::ceil(mean / sh[0]) : n_eff * row_tiles(mean, sd, sh[0]);
     const double dense_mt = dense_groups * std::ceil(static_cast<double>(dense_rows) / sh[0]);
     const double tile = ks * (sh[0] + sh[1]) + 750.0;
-    const double tiles = std::ceil((mt + dense_mt) * (ncols / sh[1]));
+    const double tiles = std::ceil((mt + dense_mt - (n_experts == 1 ? 0.0 : 0.25)) * (ncols / sh[1]));
     double cost = std::ceil(tiles / cus) * tile;
     double least = floor * (old ? 1.4 : 1.15);
     if (!old) {
@@ -2550,7 +2568,7 @@ void choose_tile(int64_t rows, int n_experts, int64_t row_bytes, int ncols, int 
     const double rounds = full * std::max(tile, stream * cus) +
                           (rest > 0.0 ? std::max(tile, stream * rest) : 0.0);
     if (dense_groups > 0) cost = rounds;
-    else if (n_experts > 1 && cost < least) cost = least;
+    else if (n_experts > 1) cost = std::max(cost, least) / (old ? 1.03 : 1.0);
     if (best == 0.0 || cost < best) {
       best = cost;
       if (units != nullptr) *units = rounds;
@@ -2729,6 +2747,19 @@ int launch_with_dense(bool swiglu, const void* A, int64_t tokens, int top_k, con
 }  // namespace
 }  // namespace hmoe
 
+extern "C" int hmoe_grouped_tile(int64_t rows_cap, int n_experts, int64_t k_bytes, int ncols, int cus,
+                                 int* rows_per_tile, int* cols_per_tile) {
+  using namespace hmoe;
+  HMOE_REQUIRE(n_experts >= 1 && n_experts <= kMaxExperts,
+               "grouped_tile: n_experts must be in [1, %d] (got %d)", kMaxExperts, n_experts);
+  HMOE_REQUIRE(rows_cap >= 1 && cus >= 1, "grouped_tile: rows_cap and cus must be >= 1");
+  HMOE_REQUIRE(k_bytes >= 128 && k_bytes % 128 == 0 && ncols >= kBN && ncols % kBN == 0,
+               "grouped_tile: k_bytes must be a multiple of 128 and ncols one of %d", kBN);
+  HMOE_REQUIRE(rows_per_tile && cols_per_tile, "grouped_tile: null pointer argument");
+  choose_tile(rows_cap, n_experts, k_bytes, ncols, cus, rows_per_tile, cols_per_tile);
+  return HMOE_OK;
+}
+
 extern "C" int hmoe_grouped_gate_up(const void* xs, const int32_t* offsets, int n_experts,
                                     int64_t rows_cap, int d_model, int d_ff,
                                     const void* w_gate_up_packed, void* h, hmoe_stream_t stream) {
@@ -2820,6 +2851,7 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
   if (rows_cap + n_shared * tokens >= (int64_t(1) << 31)) return 0;
   int dev = 0, grid = 0;
   if (persistent_grid(static_cast<hipStream_t>(stream), &grid, &dev) != HMOE_OK) return 0;
+  const bool few = rows_cap <= kJoinRows * n_experts;
   double separate = 0.0, joined = 0.0;
   for (int gemm = 0; gemm < 2; ++gemm) {
     const int64_t row_bytes = int64_t{2} * (gemm == 0 ? d_model : d_ff);
@@ -2829,13 +2861,13 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
     double routed = 0.0, dense = 0.0, both = 0.0;
     choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, 0, 0, &routed);
     if (bm == kBM) return 0;
+    if (few) continue;
     choose_tile(tokens, 1, row_bytes, ncols, grid, &bm, &bn, 0, 0, &dense);
     choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, n_shared, tokens, &both);
     separate += routed + n_shared * (dense + kLaunchUnits);
     joined += both;
   }
-  if (rows_cap <= kJoinRows * n_experts) return 1;
-  return joined * 1.03 < separate ? 1 : 0;
+  return few || joined * 1.03 < separate ? 1 : 0;
 }
 
 extern "C" int hmoe_grouped_gate_up_gather_shared(

@@ -7,6 +7,7 @@ host (so no kernel ever sees an inconsistent launch), allocates outputs with
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -328,6 +329,15 @@ def grouped_down(h: torch.Tensor, offsets: torch.Tensor, w_down: torch.Tensor,
     call("hmoe_grouped_down", _ptr(h), _ptr(offsets), N, R, F, D, _ptr(w_down), _ptr(ys),
          _stream())
     return ys
+
+
+def grouped_tile(rows: int, n_experts: int, k_bytes: int, ncols: int, cus: int) -> tuple:
+    """``(rows, columns)`` of the tile that a grouped GEMM of these sizes takes
+    (``hmoe_grouped_tile``) on a device of ``cus`` CUs."""
+    tile = (ctypes.c_int * 2)()
+    call("hmoe_grouped_tile", rows, n_experts, k_bytes, ncols, cus, ctypes.byref(tile, 0),
+         ctypes.byref(tile, ctypes.sizeof(ctypes.c_int)))
+    return tile[0], tile[1]
 
 
 def shared_joins(plan: Plan, tokens: int, w_gate_up: torch.Tensor, shared_gate_up: torch.Tensor) -> bool:

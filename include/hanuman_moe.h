@@ -217,6 +217,13 @@ int hmoe_grouped_down(const void* h, const int32_t* offsets, int n_experts,
                       int64_t rows_cap, int d_ff, int d_model,
                       const void* w_down_packed, void* ys, hmoe_stream_t stream);
 
+/* The tile that the bf16 and e4m3 grouped GEMMs (forward and data gradients)
+ * take for rows_cap rows on n_experts experts, k_bytes bytes of the reduction
+ * dimension and ncols output columns (gate/up: 2 d_ff) on a device of `cus`
+ * CUs.  A host-side query: the results do not depend on the tile. */
+int hmoe_grouped_tile(int64_t rows_cap, int n_experts, int64_t k_bytes, int ncols, int cus,
+                      int* rows_per_tile, int* cols_per_tile);
+
 /* The two GEMMs of hmoe_grouped_gate_up_gather and hmoe_grouped_down with the
  * shared experts' (moe.py:152-168; n_shared of the same d_ff, packed one after
  * another as one stack) in the same launches: shared expert i's rows follow

@@ -11,25 +11,28 @@ from hanuman_amd import kernels as K
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # T, K, N, d_model, d_ff: the chosen gate/up tile
-    (1, 1, 1, 256, 256),       # one row, one segment: 32 x 64
-    (33, 1, 1, 512, 256),      # 64 x 64, one row past a fragment
-    (129, 1, 1, 256, 384),     # several row tiles of one segment, the last of one row
-    (700, 1, 1, 2048, 1024),   # 64 x 128
-    (2000, 1, 1, 2048, 1024),  # 128 x 128
-    (4096, 1, 1, 1536, 768),   # 128 x 256
-    (3, 2, 16, 256, 256),      # fewer rows than experts, most experts empty
-    (4, 8, 64, 2048, 1024),    # 32 x 256
-    (48, 8, 64, 2048, 1024),   # 32 x 128
-    (333, 8, 80, 1536, 768),   # 64 x 256, an odd number of 128-byte steps in the down GEMM
-    (300, 3, 7, 320, 256),     # five steps (320 / 64), odd counts
+    # T, K, N, d_model, d_ff, the gate/up GEMM's tile
+    (1, 1, 1, 256, 256, (32, 64)),       # one row, one segment
+    (33, 1, 1, 512, 256, (32, 64)),      # one row past a fragment
+    (129, 1, 1, 256, 384, (32, 64)),     # several row tiles of one segment, the last of one row
+    (333, 1, 1, 1536, 768, (64, 64)),
+    (700, 1, 1, 2048, 1024, (64, 128)),
+    (2000, 1, 1, 2048, 1024, (128, 128)),
+    (4096, 1, 1, 1536, 768, (128, 256)),
+    (3, 2, 16, 256, 256, (32, 64)),      # fewer rows than experts, most experts empty
+    (16, 8, 80, 1536, 768, (32, 256)),
+    (48, 8, 64, 2048, 1024, (32, 128)),
+    (333, 8, 80, 1536, 768, (64, 256)),  # an odd number of 128-byte steps in the down GEMM
+    (300, 3, 7, 320, 256, (32, 64)),     # five steps (320 / 64), odd counts
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "T%d_K%d_N%d_D%d_F%d" % c)
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "T%d_K%d_N%d_D%d_F%d" % c[:5])
 def test_few_rows_equal_full_tiles(gpu, case):
-    T, Kk, N, D, F = case
+    T, Kk, N, D, F, tile = case
     print(f"few rows {case}", flush=True)
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    assert K.grouped_tile(T * Kk, N, 2 * D, 2 * F, cus) == tile
     g = torch.Generator(device="cpu").manual_seed(T + N)
     x = torch.randn(T, D, generator=g).to(torch.bfloat16).to(gpu)
     # a skewed choice of experts, so that segment lengths differ and some are empty

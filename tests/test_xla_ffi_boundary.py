@@ -26,6 +26,7 @@ NO_HANDLER = {
     # host-side queries, no device work
     "hmoe_abi_version",
     "hmoe_grouped_shared_joins",
+    "hmoe_grouped_tile",
 }
 
 
