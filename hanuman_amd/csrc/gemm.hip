@@ -2849,6 +2849,13 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
   if (static_cast<int64_t>(n_experts) + n_shared > kMaxExperts) return 0;
   if (tokens * d_model * 2 >= (int64_t(1) << 31)) return 0;
   if (rows_cap + n_shared * tokens >= (int64_t(1) << 31)) return 0;
+  // what launch_with_dense and the entries refuse
+  if (d_model % kBN != 0 || (2 * static_cast<int64_t>(d_ff)) % kBN != 0 || d_ff % kBK != 0) return 0;
+  const int64_t widest = std::max(d_model, d_ff);
+  if (int64_t{256} * widest * 2 >= (int64_t(1) << 31)) return 0;
+  if ((ceil_div(rows_cap + n_shared * tokens, 32) + n_experts + n_shared) *
+          (std::max<int64_t>(d_model, 2 * static_cast<int64_t>(d_ff)) / 64) >= (int64_t(1) << 31))
+    return 0;
   int dev = 0, grid = 0;
   if (persistent_grid(static_cast<hipStream_t>(stream), &grid, &dev) != HMOE_OK) return 0;
   const bool few = rows_cap <= kJoinRows * n_experts;
@@ -2856,7 +2863,6 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
   for (int gemm = 0; gemm < 2; ++gemm) {
     const int64_t row_bytes = int64_t{2} * (gemm == 0 ? d_model : d_ff);
     const int ncols = gemm == 0 ? 2 * d_ff : d_model;
-    if (ncols < 256) return 0;
     int bm = 0, bn = 0;
     double routed = 0.0, dense = 0.0, both = 0.0;
     choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, 0, 0, &routed);

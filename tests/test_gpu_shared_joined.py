@@ -1,9 +1,11 @@
 """The shared experts' tiles in the routed experts' GEMM launches, bit for bit
 against separate launches (needs an MI355X)."""
+import ctypes
+
 import pytest
 import torch
 
-from hanuman_amd import MoE
+from hanuman_amd import MoE, _lib
 from hanuman_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
@@ -47,14 +49,34 @@ def test_joined_equal_separate(gpu, case):
         assert torch.equal(shared[i], want)
 
 
+def test_no_joining_where_the_entries_refuse(gpu):
+    """The query's 0 for every size that the two entries (host checks, placeholder
+    pointers) refuse; 1 for the same sizes put right."""
+    lib, p = _lib.lib(), ctypes.c_void_p(16)
+    joins = lib.hmoe_grouped_shared_joins
+    assert joins(64, 4, 10, 256, 128, 1, None) == 1
+    for d, f in ((256, 160), (256, 100), (320, 128), (300, 128), (128, 128), (1 << 22, 128),
+                 (256, 1 << 22)):
+        rcs = {lib.hmoe_grouped_gate_up_gather_shared(p, 64, 2, p, p, 4, 10, d, f, p, p, 1, p, None)
+               if d % 64 or f % 128 or d >= 1 << 22 or f >= 1 << 22 else 0,
+               lib.hmoe_grouped_down_shared(p, p, 4, 10, 64, f, d, p, p, 1, p, None)
+               if f % 64 or d % 256 or d >= 1 << 22 or f >= 1 << 22 else 0}
+        assert rcs != {0}, (d, f)
+        assert joins(64, 4, 10, d, f, 1, None) == 0, (d, f)
+
+
 @pytest.mark.parametrize("shared,d_ff_shared", [(1, None), (2, None), (1, 512)])
 def test_module_same_result(gpu, monkeypatch, shared, d_ff_shared):
     """The module with the joined launches, and where they do not apply (another
     d_ff of the shared expert), against its separate launches."""
+    taken = []
+    rule = K.shared_joins
+    monkeypatch.setattr(K, "shared_joins", lambda *a: taken.append(rule(*a)) or taken[-1])
     layer = MoE(512, 256, 16, 4, shared, 0.02, 2.5, torch.bfloat16, 3, d_ff_shared=d_ff_shared)
     x = torch.randn(2, 19, 512, device=gpu, generator=torch.Generator(gpu).manual_seed(1))
     x = x.to(torch.bfloat16)
     with torch.no_grad():
         joined = layer(x)[0]
+        assert taken == [d_ff_shared is None]
         monkeypatch.setattr(K, "shared_joins", lambda *a: False)
         assert torch.equal(joined, layer(x)[0])
