@@ -90,6 +90,9 @@ class _PackCache:
     stride and dtype)."""
 
     def __init__(self):
+        self.clear()
+
+    def clear(self):
         self._refs = None
         self._keys = None
         self._val = None
@@ -217,6 +220,7 @@ class MoE:
         self._shared_pack = _PackCache()
         self._routed_bwd_pack = _PackCache()
         self._shared_bwd_pack = _PackCache()
+        self._backward_expected = True   # there was one since the last joint pack
 
     # ---- parameters ------------------------------------------------------
     def named_params(self) -> dict:
@@ -267,15 +271,19 @@ class MoE:
 
     def _packed_routed(self, masters=None, train: bool = False):
         """Packed routed-expert operands of ``masters`` (default: the current
-        parameters).  ``train``: a backward follows, so masters that have to be
-        packed anew are read once for its operands too."""
+        parameters).  ``train``: a backward may follow, so masters that have to
+        be packed anew are read once for its operands too; after one that no
+        backward followed, not again before there is one."""
         wg, wu, wd = masters if masters is not None else (
             self.expert_w_gate.value, self.expert_w_up.value, self.expert_w_down.value)
 
         def build():
-            if not train:
+            if not (train and self._backward_expected):
+                if train:
+                    self._routed_bwd_pack.clear()   # of masters that are gone
                 return K.pack_gate_up(wg, wu), K.pack_down(wd)
             from .backward import BackwardOperands
+            self._backward_expected = False
             gate_up, gate_up_dgrad = K.pack_gate_up_train(wg, wu)
             down, down_dgrad = K.pack_down_train(wd)
             self._routed_bwd_pack.put((wg, wu, wd),
@@ -445,6 +453,7 @@ class MoE:
         the forward's packs (rebuilt when a master changes)."""
         wg, wu, wd, swg, swu, swd = masters
         from .backward import BackwardOperands, SharedOperands
+        self._backward_expected = True
         routed = self._routed_bwd_pack.get((wg, wu, wd), lambda: BackwardOperands(wg, wu, wd))
         shared = self._shared_bwd_pack.get(
             (swg, swu, swd), lambda: SharedOperands(swg, swu, swd, self.n_shared_experts,

@@ -191,3 +191,42 @@ def test_bench_algorithmic_work_closed_forms():
     w = bench.algorithmic(wl, T * K)
     assert w["router"] == ("hbm", T * N * 4 + T * K * 8, bench.HBM_PEAK_GBS)
     assert "gate_up" not in w
+
+
+def test_backward_operands_packed_ahead_only_where_a_backward_comes(monkeypatch):
+    """A training step packs both operands of updated masters in its forward;
+    forwards that no backward follows do so once and not again, and keep none."""
+    from hanuman_amd import kernels as K
+    calls = []
+    for name in ("pack_gate_up", "pack_down", "pack_gate_up_train", "pack_down_train",
+                 "pack_gate_up_dgrad", "pack_down_dgrad"):
+        both = name.endswith("train")
+        monkeypatch.setattr(K, name, lambda *a, n=name, b=both: (
+            calls.append(n), (torch.zeros(1), torch.zeros(1)) if b else torch.zeros(1))[1])
+    m = MoE(64, 32, 2, 1, 1, 0.02, 1.0, torch.bfloat16, 0, device="cpu")
+
+    def forward(update=True, train=True):
+        calls.clear()
+        if update:
+            for p in m._params():
+                p.add_(1.0)
+        m._packed_routed(train=train)
+        return list(calls)
+
+    def backward():
+        calls.clear()
+        m._backward_operands(m._params()[1:])
+        return [c for c in calls if c != "pack_gate_up" and c != "pack_down"]
+    joint, alone = ["pack_gate_up_train", "pack_down_train"], ["pack_gate_up", "pack_down"]
+    shared = ["pack_gate_up_dgrad", "pack_down_dgrad"]
+    for _ in range(2):                       # training steps
+        assert forward() == joint and backward() == shared
+    assert forward(update=False) == [] and backward() == []
+    assert forward() == joint                # a forward alone,
+    for _ in range(2):                       # and the ones after it
+        assert forward() == alone
+        assert m._routed_bwd_pack._val is None
+    assert forward(update=False) == []
+    assert sorted(backward()) == sorted(2 * shared)   # routed and shared
+    assert forward() == joint and backward() == shared
+    assert forward(train=False) == alone and backward() == 2 * shared
