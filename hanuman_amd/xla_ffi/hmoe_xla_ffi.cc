@@ -399,6 +399,8 @@ static ffi::Error GroupedDownSharedImpl(hipStream_t stream, ffi::Buffer<ffi::BF1
                                         ffi::Buffer<ffi::S32> offsets, ffi::Buffer<ffi::U8> w,
                                         ffi::Buffer<ffi::U8> w_shared, int64_t tokens,
                                         int64_t n_shared, ffi::ResultBuffer<ffi::BF16> ys) {
+  if (Rows(*ys) != Rows(h))
+    return ffi::Error(ffi::ErrorCode::kInvalidArgument, "ys must have as many rows as h");
   return Status(hmoe_grouped_down_shared(
       h.untyped_data(), offsets.typed_data(), static_cast<int>(offsets.element_count() - 1),
       Rows(h) - n_shared * tokens, tokens, static_cast<int>(Cols(h)), static_cast<int>(Cols(*ys)),

@@ -72,6 +72,17 @@ def test_integration_training_steps_have_handlers():
     assert not sorted(bound - called), f"training steps without handlers: {sorted(bound - called)}"
 
 
+def test_joined_handlers_check_their_rows():
+    """The shared experts' rows come after the experts' in the results, which the
+    handlers size by attributes: each compares its result's rows first."""
+    text = FFI_CC.read_text()
+    for impl, checked in (("GroupedGateUpGatherSharedImpl",
+                           "if (Rows(*h) != rows_cap + n_shared * Rows(x))"),
+                          ("GroupedDownSharedImpl", "if (Rows(*ys) != Rows(h))")):
+        body = re.search(r"static ffi::Error %s\(.*?\n}\n" % impl, text, flags=re.S).group(0)
+        assert checked in body and body.index(checked) < body.index("hmoe_grouped_"), impl
+
+
 def test_jax_targets_match_handler_symbols():
     targets = _jax_targets()
     handlers = _handlers()
