@@ -305,10 +305,13 @@ def test_wgrad_gemms(gpu, R, D, F, N):
                 assert O.normwise_rel_err(dwd[e], ref) < 1e-5, ("dWd", e)
 
 
+# 128 x 64 tiles of 512 tokens below and above 256, where the split form ends:
+# 20 and 272, with token and expert remainders
+@pytest.mark.parametrize("T,D,N,tiles", [(2500, 256, 72, 20), (8200, 1024, 72, 272)])
 @pytest.mark.parametrize("x_dtype", ["bf16", "f32"])
-def test_router_dw(gpu, x_dtype):
+def test_router_dw(gpu, x_dtype, T, D, N, tiles):
+    assert tiles == D // 128 * -(-N // 64) * -(-T // 512)
     rng = np.random.default_rng(5)
-    T, D, N = 2500, 256, 72
     x = rng.standard_normal((T, D)).astype(np.float32)
     if x_dtype == "bf16":
         x = O.bf16_round(x)
