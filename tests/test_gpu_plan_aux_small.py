@@ -41,7 +41,9 @@ def test_plan_one_launch_matches_oracle(gpu, T, Kk, N, cap):
     assert (plan.perm_src.cpu().numpy()[kept:] == -1).all()
 
 
-@pytest.mark.parametrize("B,S,N,Kk", [(1, 1, 64, 8), (2, 63, 80, 8), (1, 65, 16, 2), (3, 131, 200, 4)])
+# waves with none, one, two and four tokens of a chunk
+@pytest.mark.parametrize("B,S,N,Kk", [(1, 1, 64, 8), (2, 63, 80, 8), (1, 65, 16, 2), (3, 131, 200, 4),
+                                      (5, 1, 256, 8), (2, 18, 80, 8), (1, 34, 64, 8)])
 def test_aux_losses_partial_chunks(gpu, B, S, N, Kk):
     """Sums of at most B * S * N float32 terms of one sign or nearly so, in
     another order than the oracle's float64: within 1e-5 relative."""
