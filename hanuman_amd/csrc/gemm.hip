@@ -2829,14 +2829,16 @@ namespace {
 // few rows they always gain: a shared expert alone is 16..40 tiles and two
 // launches of mostly latency.  Past kJoinRows the joined launch's last round of
 // tiles can cost more than the two launches, so there the estimates decide, by
-// a margin of 3%.  Whole layer calls, us, separate -> joined, one shared expert:
+// a margin of 3%, and of 20% where a routed GEMM alone takes 256 x 256 tiles.
+// Whole layer calls, us, separate -> joined, one shared expert:
 //   64 experts top-8, D 2048, F 1024: 1 token 124 -> 98, 48 239 -> 226, 333
 //     251 -> 235; 1500 (always 256 x 256 separate) 325, joined 378;
 //   80 experts top-8, D 1536, F 768: 48 tokens 178 -> 152, 333 187 -> 173, 900
 //     (90 rows) 213, joined 216; 1200 271 -> 237;
-//   16 experts top-2, D 1024, F 2048: 1..777 tokens 130 -> 100;
-// and two shared experts: 48 tokens of the first 278 -> 234, 333 of the second
-// 229 -> 218.
+//   16 experts top-2, D 1024, F 2048: 1..777 tokens 130 -> 100, 1000 136 -> 111;
+// two shared experts: 48 tokens of the first 278 -> 234, 333 of the second 229
+// -> 218, 1350 347 -> 312, 1000 of the third 199 -> 164; four: 1100 of the first
+// 523 -> 444.
 constexpr double kJoinRows = 48.0;
 constexpr double kLaunchUnits = 1500.0;  // a launch more, about 4 us of the estimate's units
 }  // namespace
@@ -2859,6 +2861,7 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
   int dev = 0, grid = 0;
   if (persistent_grid(static_cast<hipStream_t>(stream), &grid, &dev) != HMOE_OK) return 0;
   const bool few = rows_cap <= kJoinRows * n_experts;
+  bool full = false;  // a routed GEMM takes 256 x 256 tiles on its own
   double separate = 0.0, joined = 0.0;
   for (int gemm = 0; gemm < 2; ++gemm) {
     const int64_t row_bytes = int64_t{2} * (gemm == 0 ? d_model : d_ff);
@@ -2866,14 +2869,15 @@ extern "C" int hmoe_grouped_shared_joins(int64_t tokens, int n_experts, int64_t 
     int bm = 0, bn = 0;
     double routed = 0.0, dense = 0.0, both = 0.0;
     choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, 0, 0, &routed);
-    if (bm == kBM) return 0;
+    if (bm == kBM) full = true;
     if (few) continue;
     choose_tile(tokens, 1, row_bytes, ncols, grid, &bm, &bn, 0, 0, &dense);
     choose_tile(rows_cap, n_experts, row_bytes, ncols, grid, &bm, &bn, n_shared, tokens, &both);
     separate += routed + n_shared * (dense + kLaunchUnits);
     joined += both;
   }
-  return few || joined * 1.03 < separate ? 1 : 0;
+  if (few) return full ? 0 : 1;
+  return joined * (full ? 1.2 : 1.03) < separate ? 1 : 0;
 }
 
 extern "C" int hmoe_grouped_gate_up_gather_shared(

@@ -18,6 +18,7 @@ CASES = [
     (48, 8, 64, 2048, 1024, 2, 1.0),     # rows dropped: the experts' rows end before the shared ones
     (333, 8, 80, 1536, 768, 1, None),    # several row tiles of the shared expert, the last partial
     (300, 3, 7, 512, 128, 2, 0.5),
+    (1350, 8, 80, 1536, 768, 2, None),   # the routed GEMMs alone: 256 x 256
 ]
 
 
@@ -63,6 +64,18 @@ def test_no_joining_where_the_entries_refuse(gpu):
                if f % 64 or d % 256 or d >= 1 << 22 or f >= 1 << 22 else 0}
         assert rcs != {0}, (d, f)
         assert joins(64, 4, 10, d, f, 1, None) == 0, (d, f)
+
+
+def test_joining_rule_by_size(gpu):
+    """Few rows an expert join; many where the joined launch is clearly the
+    shorter one, also where the routed GEMM alone takes 256 x 256 tiles."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the rule's lines are those of 256 CUs")
+    joins = _lib.lib().hmoe_grouped_shared_joins
+    for tokens, n, k, d, f, shared, want in ((1, 64, 8, 2048, 1024, 1, 1), (333, 80, 8, 1536, 768, 1, 1),
+                                             (1350, 80, 8, 1536, 768, 2, 1), (1500, 64, 8, 2048, 1024, 1, 0),
+                                             (16384, 64, 8, 2048, 1024, 1, 0)):
+        assert joins(tokens, n, tokens * k, d, f, shared, None) == want, (tokens, n, shared)
 
 
 @pytest.mark.parametrize("shared,d_ff_shared", [(1, None), (2, None), (1, 512)])
